@@ -62,6 +62,7 @@ struct Frame {
   // barycentrics) plus a nonzero offset: the small-triangle keys are 32-bit
   // depth keys kept in the zbuffer itself
   int32_t narrow;
+  int32_t wide_waves;  // wavefronts per wide triangle of the binning (k_wide)
 };
 
 // floor(n / d) for 0 <= n < 2^31 with m = ceil(2^(31 + l) / d), sh = 31 + l,

@@ -13,7 +13,7 @@
 //                counted into the tiles they may cover.
 //   3. k_wide    the tile counts of triangles spanning many tiles.
 //   4. k_scan_*  exclusive scan of the per-tile counts (all scenes at once).
-//   5. k_bin     triangle ids into the tile lists (k_wide for the wide ones).
+//   5. k_bin     triangle ids into the tile lists.
 //   6. k_raster  one group per (scene, tile): stages the tile's triangle
 //                records in LDS, keeps the nearest (depth, id) key per pixel
 //                (the default primitive_chooser: argmin with first-index ties),
@@ -742,36 +742,48 @@ __global__ __launch_bounds__(kSetupThreads) __attribute__((amdgpu_waves_per_eu(8
     small_pairs(std::false_type{});
 }
 
-// Counts (BIN = false) or bins (BIN = true) the wide triangles: one wavefront
-// per triangle, its lanes striding over the triangle's tiles.  The counting
-// pass also keeps each triangle's tile-test results as a bitmap (one word per
-// 32 tiles), so the binning pass reads bits instead of testing the tiles
-// again: entry w of the wide list owns the fixed words [w * per, (w + 1) *
-// per), per = ceil(T / 32), while they fit in the pool; later entries test
-// again.
+// Counts (BIN = false) or bins (BIN = true) the wide triangles, entry w of the
+// wide list by f.wide_waves wavefronts, whose lanes take its tiles 64 at a time.
+// A step waits for its samples, so what bounds a list of few entries is the
+// longest chain of steps, not the work: with one wavefront per entry the
+// 2,040 tiles of a 960x540 frame took 32 steps (count 55 us, bin 25 us for a
+// sphere's edge-on triangles; at 4 steps the whole frame went from 161 to 88 us).  The
+// wavefronts past an entry's last tile read its range and leave, which many
+// short entries pay for, so frames of up to 256 tiles (84x84: 121) keep one.
+// The counting pass also keeps each triangle's tile-test results as a bitmap
+// (one word per 32 tiles), so the binning pass reads bits instead of testing
+// the tiles again: entry w of the wide list owns the fixed words [w * per,
+// (w + 1) * per), per = ceil(T / 32), while they fit in the pool; later entries
+// test again.
 constexpr int32_t kWideBitWords = 1 << 20;
+constexpr int32_t kWideSteps = 4;
 
+// Wavefronts per wide-list entry of a frame of T tiles.
+inline int32_t wide_waves(int32_t T) {
+  return std::min(std::max((T + 64 * kWideSteps - 1) / (64 * kWideSteps), 1), 64);
+}
+
+// wave, n_waves: the calling wavefront among those that share the list
 template <bool BIN>
-__global__ __launch_bounds__(256) void k_wide(
-    const jr_scene* __restrict__ scenes, Frame f, const float4* __restrict__ rec,
-    const Rect* __restrict__ rects, const int2* __restrict__ wide,
-    const int32_t* __restrict__ wide_count, int32_t* __restrict__ counts,
-    const int32_t* __restrict__ offsets, int32_t* __restrict__ cursor,
-    int32_t* __restrict__ bins, const float* __restrict__ samples,
-    uint32_t* __restrict__ wbits) {
+JR_DEV void wide_tiles(const jr_scene* __restrict__ scenes, const Frame& f,
+                       const float4* __restrict__ rec, const Rect* __restrict__ rects,
+                       const int2* __restrict__ wide, int32_t n, int64_t wave, int64_t n_waves,
+                       int32_t* __restrict__ counts, const int32_t* __restrict__ offsets,
+                       int32_t* __restrict__ cursor, int32_t* __restrict__ bins,
+                       const float* __restrict__ samples, uint32_t* __restrict__ wbits) {
   const int lane = threadIdx.x & 63;
-  const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const int64_t n_waves = ((int64_t)gridDim.x * blockDim.x) >> 6;
-  const int32_t n = *wide_count;
-  for (int64_t w = wave; w < n; w += n_waves) {
+  const int64_t n_items = (int64_t)n * f.wide_waves;
+  for (int64_t it = wave; it < n_items; it += n_waves) {
+    const int32_t w = (int32_t)(it / f.wide_waves), part = (int32_t)(it - (int64_t)w * f.wide_waves);
     const int2 ts = wide[w];  // (triangle, scene)
     const int32_t t = ts.x, s = ts.y;
     const Rect r = rects[t];
     const int32_t h = r.ty1 - r.ty0 + 1;
     const int32_t n_t = (r.tx1 - r.tx0 + 1) * h;
+    if (64 * part >= n_t) continue;
     const int64_t tbase = (int64_t)s * f.T;
     const int32_t per = (f.T + 31) >> 5;
-    const int32_t base = (w < kWideBitWords / per) ? (int32_t)w * per : -1;
+    const int32_t base = (w < kWideBitWords / per) ? w * per : -1;
     float4 r0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), r1 = r0, r2 = r0;
     bool sane = false;
     const float* vp = scenes[s].viewport;
@@ -781,7 +793,7 @@ __global__ __launch_bounds__(256) void k_wide(
       r2 = rec[4 * (int64_t)t + 2];
       sane = (__float_as_uint(rec[4 * (int64_t)t + 3].y) & kSane) != 0;
     }
-    for (int32_t q0 = 0; q0 < n_t; q0 += 64) {
+    for (int32_t q0 = 64 * part; q0 < n_t; q0 += 64 * f.wide_waves) {
       const int32_t q = q0 + lane;
       bool pass = false;
       if (q < n_t) {
@@ -811,6 +823,17 @@ __global__ __launch_bounds__(256) void k_wide(
       }
     }
   }
+}
+
+__global__ __launch_bounds__(256) void k_wide(
+    const jr_scene* __restrict__ scenes, Frame f, const float4* __restrict__ rec,
+    const Rect* __restrict__ rects, const int2* __restrict__ wide,
+    const int32_t* __restrict__ wide_count, int32_t* __restrict__ counts,
+    const float* __restrict__ samples, uint32_t* __restrict__ wbits) {
+  wide_tiles<false>(scenes, f, rec, rects, wide, *wide_count,
+                    ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6,
+                    ((int64_t)gridDim.x * blockDim.x) >> 6, counts, nullptr, nullptr, nullptr,
+                    samples, wbits);
 }
 
 // Stage 2: exclusive scan of n counts -> offsets (two levels, 2048 per block).
@@ -882,28 +905,40 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_add(
     if (base + q < n) offsets[base + q] += add;
 }
 
-// Stage 3: write triangle ids into the tile lists.
+// Stage 3: write triangle ids into the tile lists: the first list_groups
+// workgroups those of k_setup's list, the others the wide triangles' (one
+// launch, so that the two run beside each other and one launch of about 5 us is
+// saved: 60 frames of 480x270 232.7 -> 217.0 us, a cube 44.6 -> 42.8 us).
 // One (triangle, tile) pair per lane-step: the wavefront's binned triangles'
 // set mask bits are numbered by a prefix sum of their counts and spread over
 // the lanes, so every step issues up to 64 independent slot claims instead of
 // each lane claiming its tiles one after another.  All staging is
 // wavefront-local.
 __global__ __launch_bounds__(256) void k_bin(
-    Frame f, const Rect* __restrict__ rects,
-    const int32_t* __restrict__ offsets, int32_t* __restrict__ cursor,
-    int32_t* __restrict__ bins, const uint32_t* __restrict__ masks,
-    const int2* __restrict__ blist, const int32_t* __restrict__ blist_n) {
+    const jr_scene* __restrict__ scenes, Frame f, const float4* __restrict__ rec,
+    const Rect* __restrict__ rects, const int32_t* __restrict__ offsets,
+    int32_t* __restrict__ cursor, int32_t* __restrict__ bins, const uint32_t* __restrict__ masks,
+    const int2* __restrict__ blist, const int2* __restrict__ wide,
+    const int32_t* __restrict__ wide_count, const float* __restrict__ samples,
+    uint32_t* __restrict__ wbits, int32_t list_groups) {
   __shared__ int4 own[256];  // tile range (tx0, ty0, height in tiles) and s * T
   __shared__ int32_t own_t[256];
   __shared__ uint32_t own_m[256];
   __shared__ int32_t own_off[256];  // exclusive prefix sum of the bit counts
   __shared__ int8_t mark[256];      // wave_owner scratch, 64 per wavefront
+  if ((int32_t)blockIdx.x >= list_groups) {
+    const int64_t first = (int64_t)((int32_t)blockIdx.x - list_groups) * blockDim.x;
+    wide_tiles<true>(scenes, f, rec, rects, wide, *wide_count, (first + threadIdx.x) >> 6,
+                     ((int64_t)((int32_t)gridDim.x - list_groups) * blockDim.x) >> 6, nullptr,
+                     offsets, cursor, bins, samples, wbits);
+    return;
+  }
   const int lane = threadIdx.x & 63;
   const int wbase = threadIdx.x & ~63;
-  const int32_t n = *blist_n;
+  const int32_t n = wide_count[kBinListAt];
   // the wavefronts stride over k_setup's list, 64 entries at a time
   const int32_t wave = (int32_t)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-  const int32_t n_waves = (int32_t)((gridDim.x * blockDim.x) >> 6);
+  const int32_t n_waves = (int32_t)((list_groups * blockDim.x) >> 6);
   for (int32_t first = wave * 64; first < n; first += n_waves * 64) {
     const int32_t i = first + lane;
     int32_t n_b = 0;
@@ -1627,6 +1662,7 @@ Frame dev_frame(const jr_frame* fr, bool narrow) {
   f.n_scenes = fr->n_scenes;
   f.capacity = fr->bin_capacity;
   f.narrow = narrow;
+  f.wide_waves = wide_waves(f.T);
   return f;
 }
 
@@ -1886,7 +1922,11 @@ int32_t forward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* sc
   int32_t* wide_count = misc + 2;
   uint32_t* wbits = reinterpret_cast<uint32_t*>(ws + L.wbits);
   int2* blist = reinterpret_cast<int2*>(ws + L.blist);
-  const unsigned wide_grid = 8192;  // 32768 wavefronts stride over the wide list
+  // the wavefronts striding over the wide list: at most one for each part of
+  // an entry and 32768 in all (a cube's 12 triangles need no 8192 workgroups,
+  // which took 3.5 us to start and end)
+  const unsigned wide_groups =
+      (unsigned)std::min<int64_t>(((int64_t)in->n_tris * f.wide_waves + 3) / 4, 8192);
 
   // a binning-only call is timed too (its raster stage then takes no time)
   StageTimer timer(st, timed && fr->part != JR_PART_RASTER);
@@ -1914,8 +1954,8 @@ int32_t forward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* sc
                        masks, wave_scene, blist);
   timer.mark(2);
   if (n_tris > 0)
-    hipLaunchKernelGGL(k_wide<false>, dim3(wide_grid), dim3(256), 0, st, scenes, f, rec,
-                       rects, wide, wide_count, counts, offsets, cursor, bins, samples, wbits);
+    hipLaunchKernelGGL(k_wide, dim3(wide_groups), dim3(256), 0, st, scenes, f, rec, rects, wide,
+                       wide_count, counts, samples, wbits);
   timer.mark(3);
   hipLaunchKernelGGL(k_scan_local, dim3((unsigned)std::max<int64_t>(L.nblk, 1)),
                      dim3(kScanThreads), 0, st, counts, offsets, block_sums, L.n_tiles);
@@ -1925,11 +1965,10 @@ int32_t forward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* sc
                      dim3(kScanThreads), 0, st, offsets, block_sums, L.n_tiles);
   timer.mark(4);
   if (n_tris > 0) {
-    hipLaunchKernelGGL(k_bin, dim3((unsigned)std::min((n_tris + 255) / 256, 2048)), dim3(256), 0,
-                       st, f, rects, offsets, cursor, bins, masks, blist,
-                       wide_count + kBinListAt);
-    hipLaunchKernelGGL(k_wide<true>, dim3(wide_grid), dim3(256), 0, st, scenes, f, rec,
-                       rects, wide, wide_count, counts, offsets, cursor, bins, samples, wbits);
+    const int32_t list_groups = std::min((n_tris + 255) / 256, 2048);
+    hipLaunchKernelGGL(k_bin, dim3((unsigned)list_groups + wide_groups), dim3(256), 0, st, scenes,
+                       f, rec, rects, offsets, cursor, bins, masks, blist, wide, wide_count,
+                       samples, wbits, list_groups);
   }
   timer.mark(5);
   }

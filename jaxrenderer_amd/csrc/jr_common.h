@@ -63,6 +63,7 @@ struct Frame {
   // depth keys kept in the zbuffer itself
   int32_t narrow;
   int32_t wide_waves;  // wavefronts per wide triangle of the binning (k_wide)
+  int64_t keys_at;     // offset of the key buffer in its workspace
 };
 
 // floor(n / d) for 0 <= n < 2^31 with m = ceil(2^(31 + l) / d), sh = 31 + l,

@@ -12,7 +12,7 @@
 //                small triangles resolved into the key buffer, the others
 //                counted into the tiles they may cover.
 //   3. k_wide    the tile counts of triangles spanning many tiles.
-//   4. k_scan_*  exclusive scan of the per-tile counts (all scenes at once).
+//   4. k_offsets a list segment for every tile (all scenes at once).
 //   5. k_bin     triangle ids into the tile lists.
 //   6. k_raster  one group per (scene, tile): stages the tile's triangle
 //                records in LDS, keeps the nearest (depth, id) key per pixel
@@ -277,7 +277,7 @@ JR_DEV bool has_nan_column(const float4& r) {
 // wide form's k_clear marks it stale), or the epoch running out.  The fill
 // value ~0 has tag 0xFFFFFFFF, which no epoch >= 1 produces.
 constexpr int kKsMagic = 0, kKsPixLo = 1, kKsPixHi = 2, kKsOffLo = 3, kKsOffHi = 4,
-              kKsEpoch = 5, kKsFill = 6;
+              kKsEpoch = 5;
 constexpr uint32_t kKeyMagic = 0x6b657973u;
 
 JR_DEV uint64_t tagged_key(uint32_t key, uint32_t tag) {
@@ -287,26 +287,34 @@ JR_DEV uint32_t untag_key(uint64_t k, uint32_t tag) {
   return (uint32_t)(k >> 32) == tag ? (uint32_t)k : ~0u;
 }
 
-// Before a narrow binning: the next epoch, or a full fill of the key buffer
-// (by k_clear) with epoch 1 when the state does not describe the buffer.
-__global__ void k_keys_prepare(uint32_t* __restrict__ ks, int64_t n_pix, int64_t keys_at) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  const uint32_t lo = (uint32_t)n_pix, hi = (uint32_t)((uint64_t)n_pix >> 32);
-  const uint32_t olo = (uint32_t)keys_at, ohi = (uint32_t)((uint64_t)keys_at >> 32);
+// The epoch of a narrow binning, and whether its key buffer has to be filled
+// first (then epoch 1): a function of the state that the last binning left,
+// which k_clear and k_setup each evaluate and k_offsets, after both, advances
+// (a launch of its own for that took 3 to 5 us of every call).
+struct KeyEpoch {
+  uint32_t epoch;
+  bool fill;
+};
+JR_DEV KeyEpoch next_epoch(const uint32_t* __restrict__ ks, const Frame& f) {
+  const uint64_t n = (uint64_t)f.W * (uint64_t)f.H * (uint64_t)f.n_scenes, at = (uint64_t)f.keys_at;
   const uint32_t e = ks[kKsEpoch];
-  const bool ok = ks[kKsMagic] == kKeyMagic && ks[kKsPixLo] == lo && ks[kKsPixHi] == hi &&
-                  ks[kKsOffLo] == olo && ks[kKsOffHi] == ohi && e >= 1u && e < 0xFFFFFFFEu;
-  ks[kKsFill] = ok ? 0u : 1u;
-  ks[kKsEpoch] = ok ? e + 1u : 1u;
+  const bool ok = ks[kKsMagic] == kKeyMagic && ks[kKsPixLo] == (uint32_t)n &&
+                  ks[kKsPixHi] == (uint32_t)(n >> 32) && ks[kKsOffLo] == (uint32_t)at &&
+                  ks[kKsOffHi] == (uint32_t)(at >> 32) && e >= 1u && e < 0xFFFFFFFEu;
+  return {ok ? e + 1u : 1u, !ok};
+}
+JR_DEV void advance_epoch(uint32_t* __restrict__ ks, const Frame& f) {
+  const uint64_t n = (uint64_t)f.W * (uint64_t)f.H * (uint64_t)f.n_scenes, at = (uint64_t)f.keys_at;
+  ks[kKsEpoch] = next_epoch(ks, f).epoch;
   ks[kKsMagic] = kKeyMagic;
-  ks[kKsPixLo] = lo;
-  ks[kKsPixHi] = hi;
-  ks[kKsOffLo] = olo;
-  ks[kKsOffHi] = ohi;
+  ks[kKsPixLo] = (uint32_t)n;
+  ks[kKsPixHi] = (uint32_t)(n >> 32);
+  ks[kKsOffLo] = (uint32_t)at;
+  ks[kKsOffHi] = (uint32_t)(at >> 32);
 }
 
 // Clears the tile counters (n32 int32), sets the n64 per-pixel keys to "no
-// candidate" (the narrow form: only when k_keys_prepare asked for a fill; the
+// candidate" (the narrow form: only when next_epoch asks for a fill; the
 // wide form: always, and the key state no longer describes the buffer) and
 // fills every scene's sample table: the NDC coordinates pix_x(i) for i < W
 // followed by pix_y(j) for j < H.
@@ -332,7 +340,7 @@ __global__ void k_clear(int32_t* __restrict__ p32, int64_t n32, uint64_t* __rest
   }
   for (int64_t i = first; i < n32; i += stride) p32[i] = 0;
   if (f.narrow) {
-    if (ks[kKsFill] == 0u) n64 = 0;
+    if (!next_epoch(ks, f).fill) n64 = 0;
   } else if (first == 0) {
     ks[kKsMagic] = 0u;
   }
@@ -696,7 +704,7 @@ __global__ __launch_bounds__(kSetupThreads) __attribute__((amdgpu_waves_per_eu(8
     vz1 = scenes[s_lo].viewport[11];
     __syncthreads();
   }
-  const uint32_t tag = f.narrow ? ~ks[kKsEpoch] : 0u;  // this binning's key tag
+  const uint32_t tag = f.narrow ? ~next_epoch(ks, f).epoch : 0u;  // this binning's key tag
   // the tile raster's exact per-pixel arithmetic for every (triangle, pixel)
   auto small_pairs = [&](auto from_lds) {
     constexpr bool LDS = decltype(from_lds)::value;
@@ -808,7 +816,7 @@ JR_DEV void wide_tiles(const jr_scene* __restrict__ scenes, const Frame& f,
           const int64_t gt = tbase + tx * f.tiles_y + ty;
           if (BIN) {
             const int64_t pos = (int64_t)offsets[gt] + atomicAdd(cursor + gt, 1);
-            if (pos < f.capacity) bins[pos] = t;
+            if ((uint64_t)pos < (uint64_t)f.capacity) bins[pos] = t;
           } else {
             atomicAdd(counts + gt, 1);
           }
@@ -836,73 +844,55 @@ __global__ __launch_bounds__(256) void k_wide(
                     samples, wbits);
 }
 
-// Stage 2: exclusive scan of n counts -> offsets (two levels, 2048 per block).
-constexpr int kScanThreads = 256;
-constexpr int kScanPer = 8;
-constexpr int kScanBlock = kScanThreads * kScanPer;
+// Stage 2: a segment of the list buffer for each of n tiles, as long as its
+// count, and the sum of all counts in *total (zero before).  A workgroup sums
+// its 2048 counts and takes that much with one atomic, so segments ascend
+// inside a workgroup and the workgroups' come in any order: a tile needs a
+// segment of its own, not a place in a scan over all tiles, and this is one
+// launch where a scan takes three dependent ones (a cube's frame 42.2 -> 37.9
+// us, 200 walkers' 186.7 -> 177.8 us).
+constexpr int kOffThreads = 256;
+constexpr int kOffPer = 8;
+constexpr int kOffBlock = kOffThreads * kOffPer;
 
-JR_DEV int32_t block_excl_scan(int32_t v, int32_t* lds, int32_t* total) {
-  const int tid = threadIdx.x;
-  lds[tid] = v;
-  __syncthreads();
-  for (int off = 1; off < kScanThreads; off <<= 1) {
-    const int32_t add = (tid >= off) ? lds[tid - off] : 0;
-    __syncthreads();
-    lds[tid] += add;
-    __syncthreads();
-  }
-  const int32_t incl = lds[tid];
-  *total = lds[kScanThreads - 1];
-  __syncthreads();
-  return incl - v;
-}
-
-__global__ __launch_bounds__(kScanThreads) void k_scan_local(
-    const int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
-    int32_t* __restrict__ block_sums, int64_t n) {
-  __shared__ int32_t lds[kScanThreads];
-  const int64_t base = (int64_t)blockIdx.x * kScanBlock + threadIdx.x * kScanPer;
-  int32_t v[kScanPer];
+__global__ __launch_bounds__(kOffThreads) void k_offsets(const int32_t* __restrict__ counts,
+                                                         int32_t* __restrict__ offsets, int64_t n,
+                                                         int32_t* __restrict__ total,
+                                                         uint32_t* __restrict__ ks, Frame f) {
+  __shared__ int32_t wave_total[kOffThreads / 64];
+  __shared__ int32_t first;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t base = (int64_t)blockIdx.x * kOffBlock + threadIdx.x * kOffPer;
+  int32_t v[kOffPer];
   int32_t sum = 0;
 #pragma unroll
-  for (int q = 0; q < kScanPer; ++q) {
+  for (int q = 0; q < kOffPer; ++q) {
     v[q] = (base + q < n) ? counts[base + q] : 0;
     sum += v[q];
   }
-  int32_t total;
-  int32_t run = block_excl_scan(sum, lds, &total);
+  int32_t incl = sum;
 #pragma unroll
-  for (int q = 0; q < kScanPer; ++q) {
+  for (int d = 1; d < 64; d <<= 1) {
+    const int32_t up = __shfl_up(incl, d, 64);
+    if (lane >= d) incl += up;
+  }
+  if (lane == 63) wave_total[wave] = incl;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int32_t all = 0;
+#pragma unroll
+    for (int w = 0; w < kOffThreads / 64; ++w) all += wave_total[w];
+    first = all != 0 ? atomicAdd(total, all) : 0;
+    if (f.narrow && blockIdx.x == 0) advance_epoch(ks, f);
+  }
+  __syncthreads();
+  int32_t run = first + incl - sum;
+  for (int w = 0; w < wave; ++w) run += wave_total[w];
+#pragma unroll
+  for (int q = 0; q < kOffPer; ++q) {
     if (base + q < n) offsets[base + q] = run;
     run += v[q];
   }
-  if (threadIdx.x == 0) block_sums[blockIdx.x] = total;
-}
-
-// Scans the block sums in place (one group, any count) and stores the grand
-// total in *total_out.
-__global__ __launch_bounds__(kScanThreads) void k_scan_top(
-    int32_t* __restrict__ block_sums, int64_t nblk, int32_t* __restrict__ total_out) {
-  __shared__ int32_t lds[kScanThreads];
-  int32_t carry = 0;
-  for (int64_t c = 0; c < nblk; c += kScanThreads) {
-    const int64_t i = c + threadIdx.x;
-    const int32_t v = (i < nblk) ? block_sums[i] : 0;
-    int32_t total;
-    const int32_t ex = block_excl_scan(v, lds, &total);
-    if (i < nblk) block_sums[i] = carry + ex;
-    carry += total;
-  }
-  if (threadIdx.x == 0) *total_out = carry;
-}
-
-__global__ __launch_bounds__(kScanThreads) void k_scan_add(
-    int32_t* __restrict__ offsets, const int32_t* __restrict__ block_sums,
-    int64_t n) {
-  const int64_t base = (int64_t)blockIdx.x * kScanBlock;
-  const int32_t add = block_sums[blockIdx.x];
-  for (int q = threadIdx.x; q < kScanBlock; q += kScanThreads)
-    if (base + q < n) offsets[base + q] += add;
 }
 
 // Stage 3: write triangle ids into the tile lists: the first list_groups
@@ -972,7 +962,7 @@ __global__ __launch_bounds__(256) void k_bin(
       const int32_t tx = box.x + dq, ty = box.y + (q - dq * box.z);
       const int64_t gt = (int64_t)box.w + tx * f.tiles_y + ty;
       const int64_t pos = (int64_t)offsets[gt] + atomicAdd(cursor + gt, 1);
-      if (pos < f.capacity) bins[pos] = own_t[o];
+      if ((uint64_t)pos < (uint64_t)f.capacity) bins[pos] = own_t[o];
     }
     tile_sync<true>();  // the entries' staging is rewritten by the next step
   }
@@ -1431,7 +1421,7 @@ JR_DEV void raster_tile(const RasterArgs& a, int64_t gt, float4* lds_rec,
 
   const int32_t cnt = a.counts[gt];
   const int64_t start = a.offsets[gt];
-  const bool overflow = start + cnt > f.capacity;
+  const bool overflow = start < 0 || start + cnt > f.capacity;
   // overflowing tile lists fall back to every triangle of the scene
   const int32_t n_items = overflow ? (sc.tri_end - sc.tri_begin) : cnt;
   for (int32_t base = 0; base < n_items; base += NT) {
@@ -1632,7 +1622,7 @@ constexpr int64_t kAlign = 256;
 int64_t align_up(int64_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 
 struct WsLayout {
-  int64_t rec, rects, counts, cursor, offsets, block_sums, misc, keys, kstate, wide, samples,
+  int64_t rec, rects, counts, cursor, offsets, misc, keys, kstate, wide, samples,
       masks, wave_scene, wbits, bins, blist, total;
   int64_t n_tiles, nblk, n_pix;
 };
@@ -1663,6 +1653,7 @@ Frame dev_frame(const jr_frame* fr, bool narrow) {
   f.capacity = fr->bin_capacity;
   f.narrow = narrow;
   f.wide_waves = wide_waves(f.T);
+  f.keys_at = 0;
   return f;
 }
 
@@ -1681,17 +1672,16 @@ WsLayout ws_layout(const jr_frame* fr, int32_t n_tris) {
   const int64_t tiles_x = (fr->width + fr->tile_w - 1) / fr->tile_w;
   const int64_t tiles_y = (fr->height + fr->tile_h - 1) / fr->tile_h;
   L.n_tiles = tiles_x * tiles_y * (int64_t)fr->n_scenes;
-  L.nblk = (L.n_tiles + kScanBlock - 1) / kScanBlock;
+  L.nblk = (L.n_tiles + kOffBlock - 1) / kOffBlock;
   int64_t o = 0;
-  L.kstate = o;     o += align_up(64);   // key state (k_keys_prepare): first in every layout
+  L.kstate = o;     o += align_up(64);   // key state (next_epoch): first in every layout
   L.rec = o;        o += align_up(64 * (int64_t)std::max(n_tris, 1));
   L.rects = o;      o += align_up(16 * (int64_t)std::max(n_tris, 1));
   L.counts = o;     o += align_up(4 * L.n_tiles);
   L.cursor = o;     o += align_up(4 * L.n_tiles);
   L.misc = o;       o += align_up(256);  // [0] total pairs, [1] work counter, [2] wide count,
                                          // [2 + kBinListAt] k_bin's list length
-  L.offsets = o;    o += align_up(4 * (L.n_tiles + 1));
-  L.block_sums = o; o += align_up(4 * std::max<int64_t>(L.nblk, 1));
+  L.offsets = o;    o += align_up(4 * L.n_tiles);
   L.n_pix = (int64_t)fr->width * fr->height * fr->n_scenes;
   L.keys = o;       o += align_up(8 * L.n_pix);
   L.wide = o;       o += align_up(8 * (int64_t)std::max(n_tris, 1));
@@ -1903,7 +1893,8 @@ namespace jr {
 int32_t forward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* scenes,
                      jr_outputs* out, char* ws, const WsLayout& L, hipStream_t st,
                      bool timed) {
-  const Frame f = dev_frame(fr, narrow_form(fr, out->prim_id || out->bary));
+  Frame f = dev_frame(fr, narrow_form(fr, out->prim_id || out->bary));
+  f.keys_at = L.keys;
 
   float4* rec = reinterpret_cast<float4*>(ws + L.rec);
   Rect* rects = reinterpret_cast<Rect*>(ws + L.rects);
@@ -1911,7 +1902,6 @@ int32_t forward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* sc
   int32_t* cursor = reinterpret_cast<int32_t*>(ws + L.cursor);
   int32_t* misc = reinterpret_cast<int32_t*>(ws + L.misc);
   int32_t* offsets = reinterpret_cast<int32_t*>(ws + L.offsets);
-  int32_t* block_sums = reinterpret_cast<int32_t*>(ws + L.block_sums);
   int32_t* bins = reinterpret_cast<int32_t*>(ws + L.bins);
   uint64_t* keys = reinterpret_cast<uint64_t*>(ws + L.keys);
   uint32_t* kstate = reinterpret_cast<uint32_t*>(ws + L.kstate);
@@ -1941,8 +1931,6 @@ int32_t forward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* sc
   const int64_t nclr = std::max(std::max(nz, f.narrow ? std::min<int64_t>(L.n_pix, 1 << 20)
                                                       : L.n_pix),
                                 (int64_t)(f.W + f.H) * f.n_scenes);
-  if (f.narrow)
-    hipLaunchKernelGGL(k_keys_prepare, dim3(1), dim3(64), 0, st, kstate, L.n_pix, L.keys);
   hipLaunchKernelGGL(k_clear, dim3((unsigned)std::min<int64_t>((nclr + 255) / 256, 8192)),
                      dim3(256), 0, st, counts, nz, keys, L.n_pix, kstate, scenes, f, samples,
                      wave_scene, in->n_tris);
@@ -1957,12 +1945,8 @@ int32_t forward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* sc
     hipLaunchKernelGGL(k_wide, dim3(wide_groups), dim3(256), 0, st, scenes, f, rec, rects, wide,
                        wide_count, counts, samples, wbits);
   timer.mark(3);
-  hipLaunchKernelGGL(k_scan_local, dim3((unsigned)std::max<int64_t>(L.nblk, 1)),
-                     dim3(kScanThreads), 0, st, counts, offsets, block_sums, L.n_tiles);
-  hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(kScanThreads), 0, st, block_sums,
-                     L.nblk, misc);
-  hipLaunchKernelGGL(k_scan_add, dim3((unsigned)std::max<int64_t>(L.nblk, 1)),
-                     dim3(kScanThreads), 0, st, offsets, block_sums, L.n_tiles);
+  hipLaunchKernelGGL(k_offsets, dim3((unsigned)L.nblk), dim3(kOffThreads), 0, st, counts, offsets,
+                     L.n_tiles, misc, kstate, f);
   timer.mark(4);
   if (n_tris > 0) {
     const int32_t list_groups = std::min((n_tris + 255) / 256, 2048);

@@ -24,8 +24,8 @@
 //                 per pixel, shading backward (texture / specular gradients
 //                 summed per texel in LDS), the visibility backward (dL/dM^-1,
 //                 dL/dz_clip, per-corner varying cotangents) summed per
-//                 triangle in LDS, then one set of global atomics per
-//                 (tile, triangle) and per (tile, texel)
+//                 triangle across lanes and in LDS, then one set of global
+//                 atomics per (tile, triangle) and per (tile, texel)
 //   k_bwd_tris    one thread per triangle, the touched ones packed together:
 //                 M^-1 -> M -> clip -> positions and the vertex stage of each
 //                 corner (normals, colours, light, camera matrices)
@@ -64,34 +64,31 @@ inline int acc_floats(int shader) {
   return shader == JR_SHADER_PHONG_DARBOUX ? AccOf<JR_SHADER_PHONG_DARBOUX>::N : kAcc;
 }
 
-// per-scene gradients reduced in k_bwd_pixels
+// per-scene sums of k_bwd_pixels, three floats each; a shader has the first
+// scene_sums() of them.  S_DIR is the light direction that its fragment stage
+// normalises: light_dir_eye of the reflection shaders, light_direction of phong
+// and phong_darboux.  The reflection shaders sum c diff and c spec (c: the
+// cotangent times the texel, times the shadow factor) into S_DIFFUSE and
+// S_SPECULAR, from which the gradients of diffuse, specular and the light's colour
+// follow; phong and phong_darboux sum the last one in S_DIFFUSE's place.
 enum {
-  S_LIGHT_COLOUR = 0,
-  S_LIGHT_DIR_EYE = 3,
-  S_AMBIENT = 6,
-  S_DIFFUSE = 9,
-  S_SPECULAR = 12,
-  S_STRENGTH = 15,
-  S_LIGHT_DIR = 18,
-  S_VP00 = 21,
-  S_VP03 = 22,
-  S_VP11 = 23,
-  S_VP13 = 24,
-  S_VP22 = 25,
-  S_VP23 = 26,
-  S_COUNT = 27
+  S_DIR = 0,
+  S_LIGHT_COLOUR = 3,
+  S_DIFFUSE = 3,
+  S_SPECULAR = 6,
+  S_AMBIENT = 9,
+  S_STRENGTH = 12,
+  S_COUNT = 15
 };
-
-__device__ __constant__ int kSceneSlot[S_COUNT] = {
-    JR_DSCENE_LIGHT_COLOUR, JR_DSCENE_LIGHT_COLOUR + 1, JR_DSCENE_LIGHT_COLOUR + 2,
-    JR_DSCENE_LIGHT_DIR_EYE, JR_DSCENE_LIGHT_DIR_EYE + 1, JR_DSCENE_LIGHT_DIR_EYE + 2,
-    JR_DSCENE_AMBIENT, JR_DSCENE_AMBIENT + 1, JR_DSCENE_AMBIENT + 2,
-    JR_DSCENE_DIFFUSE, JR_DSCENE_DIFFUSE + 1, JR_DSCENE_DIFFUSE + 2,
-    JR_DSCENE_SPECULAR, JR_DSCENE_SPECULAR + 1, JR_DSCENE_SPECULAR + 2,
-    JR_DSCENE_SHADOW_STRENGTH, JR_DSCENE_SHADOW_STRENGTH + 1, JR_DSCENE_SHADOW_STRENGTH + 2,
-    JR_DSCENE_LIGHT_DIRECTION, JR_DSCENE_LIGHT_DIRECTION + 1, JR_DSCENE_LIGHT_DIRECTION + 2,
-    JR_DSCENE_VIEWPORT + 0, JR_DSCENE_VIEWPORT + 3, JR_DSCENE_VIEWPORT + 5,
-    JR_DSCENE_VIEWPORT + 7, JR_DSCENE_VIEWPORT + 10, JR_DSCENE_VIEWPORT + 11};
+constexpr bool reflects(int shader) {
+  return shader == JR_SHADER_PHONG_REFLECTION || shader == JR_SHADER_PHONG_REFLECTION_SHADOW;
+}
+constexpr int scene_sums(int shader) {
+  return shader == JR_SHADER_PHONG_REFLECTION_SHADOW ? S_COUNT
+         : shader == JR_SHADER_PHONG_REFLECTION      ? S_STRENGTH
+         : shader == JR_SHADER_PHONG || shader == JR_SHADER_PHONG_DARBOUX ? S_SPECULAR
+                                                                          : 0;
+}
 
 // y = v / |v|: dv = (dy - y (y . dy)) / |v|
 JR_DEV void normalise_bwd(const float v[3], const float dy[3], float dv[3]) {
@@ -109,151 +106,119 @@ JR_DEV float max_grad(float a, float b) {
   return a > b ? 1.0f : (a == b ? 0.5f : 0.0f);
 }
 
+// What one pixel hands to the sums: the cotangent dn of its interpolated
+// 3-vector, the texel, specular-map and normal-map entry its gradients land on
+// (u < 0: none) with the gradients, and phong_darboux's cotangents of the face's
+// NDC corners and their uvs.
+template <int SHADER>
 struct PixGrad {
-  float db[3];
-  float dvar[3][3];
-  float sg[S_COUNT];
-  // the texel, specular-map and normal-map entry this pixel's gradient lands
-  // on (-1: none); scattered after the per-pixel work, with the wavefront
-  // converged
-  int64_t tex_at, spec_at, nmap_at;
-  int32_t tex_n;
-  float tex_g[3], spec_g, nmap_g[3];
-  // phong_darboux: cotangents of the face's NDC corners and their uvs
-  float dtri[9], dtuv[6];
+  static constexpr bool kDarboux = SHADER == JR_SHADER_PHONG_DARBOUX;
+  float dn[3];
+  int32_t u, v;            // diffuse texel
+  int32_t us, vs;          // specular-map or normal-map entry
+  float tex_g[3], spec_g, nmap_g[kDarboux ? 3 : 1];
+  float more[kDarboux ? 15 : 1];
+  JR_DEV PixGrad() {
+    dn[0] = dn[1] = dn[2] = 0.0f;
+    u = us = -1;
+    v = vs = 0;
+    tex_g[0] = tex_g[1] = tex_g[2] = spec_g = 0.0f;
+    nmap_g[0] = 0.0f;
+    if constexpr (kDarboux) {
+      nmap_g[1] = nmap_g[2] = 0.0f;
+#pragma unroll
+      for (int k = 0; k < 15; ++k) more[k] = 0.0f;
+    }
+  }
 };
 
-// A texel lookup transposes to an add at the same (already clamped) index.
-JR_DEV void add_tex(PixGrad& pg, int64_t base, int32_t th, int32_t tc, int32_t u, int32_t v,
-                    const float g[3]) {
-  pg.tex_at = base + ((int64_t)u * th + v) * tc;
-  if (tc > 1) {
-    pg.tex_n = 3;
-    pg.tex_g[0] = g[0];
-    pg.tex_g[1] = g[1];
-    pg.tex_g[2] = g[2];
-  } else {
-    pg.tex_n = 1;
-    pg.tex_g[0] = (g[0] + g[1]) + g[2];
-  }
-}
-
+// Reverse of Varyings<SHADER>::pixel.  vary: the corner stage; n: interp() of its
+// first 9 floats; l: Varyings<SHADER>::scene_terms; sg: the lane's per-scene sums.
 template <int SHADER>
 struct ShadeBwd;
 
 template <>
-struct ShadeBwd<JR_SHADER_DEPTH> {
-  static JR_DEV void run(const jr_inputs&, const jr_scene&, const jr_grads&, const Corner&,
-                         const float*, const float*, PixGrad&, int) {}
-};
-
-// The shaders whose corner stage a tile stages once per triangle
-// (Varyings<SHADER>): run() computes it, run_v() takes it.
-template <int SHADER>
-struct CornerBwd {
-  static JR_DEV void run(const jr_inputs& in, const jr_scene& sc, const jr_grads& gr,
-                         const Corner& c, const float b[3], const float dcol[3], PixGrad& g,
-                         int scene) {
-    float v[Varyings<SHADER>::N];
-    Varyings<SHADER>::corners(in, sc, c, v);
-    ShadeBwd<SHADER>::run_v(in, sc, gr, v, b, dcol, g, scene);
-  }
-};
+struct ShadeBwd<JR_SHADER_DEPTH> {};
 
 // shaders/gouraud.py:90-124: col = sum_k b_k col_k
 template <>
-struct ShadeBwd<JR_SHADER_GOURAUD> : CornerBwd<JR_SHADER_GOURAUD> {
-  // v: the three corners' lit colours
-  static JR_DEV void run_v(const jr_inputs&, const jr_scene&, const jr_grads&,
-                           const float* v, const float b[3], const float dcol[3], PixGrad& g,
-                           int) {
-    for (int k = 0; k < 3; ++k) {
-      g.db[k] = dot3(dcol, v + 3 * k);
-      for (int q = 0; q < 3; ++q) g.dvar[k][q] = b[k] * dcol[q];
-    }
+struct ShadeBwd<JR_SHADER_GOURAUD> {
+  static JR_DEV void run(const jr_inputs&, const jr_scene&, const jr_grads&, const float*,
+                         const float[3], const float[3], const float[3],
+                         const float dcol[3], PixGrad<JR_SHADER_GOURAUD>& g, float*, int) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) g.dn[q] = dcol[q];
   }
 };
 
+// Texel of the wrapping shaders: floor(uv) mod the map's shape.
+JR_DEV void wrapped_texel(const jr_scene& sc, const float* uvv, const float b[3], int32_t* u,
+                          int32_t* v) {
+  const float uu = interp(b, uvv[0], uvv[2], uvv[4]);
+  const float vv = interp(b, uvv[1], uvv[3], uvv[5]);
+  *u = floor_mod(f2i_sat(floorf(uu)), sc.tex_w);
+  *v = floor_mod(f2i_sat(floorf(vv)), sc.tex_h);
+}
+
 // shaders/gouraud_texture.py:103-144: col = texture[uv] * sum_k b_k lc_k
 template <>
-struct ShadeBwd<JR_SHADER_GOURAUD_TEXTURE> : CornerBwd<JR_SHADER_GOURAUD_TEXTURE> {
-  // v: the corners' light colours lc_k (3 x 3), then their uvs (3 x 2)
-  static JR_DEV void run_v(const jr_inputs& in, const jr_scene& sc, const jr_grads&,
-                           const float* v, const float b[3], const float dcol[3], PixGrad& g,
-                           int) {
-    const float* uvv = v + 9;
-    float light[3];
-    for (int q = 0; q < 3; ++q) light[q] = interp(b, v[q], v[3 + q], v[6 + q]);
-    const float uu = interp(b, uvv[0], uvv[2], uvv[4]);
-    const float vv = interp(b, uvv[1], uvv[3], uvv[5]);
-    const int32_t u = floor_mod(f2i_sat(floorf(uu)), sc.tex_w);
-    const int32_t t = floor_mod(f2i_sat(floorf(vv)), sc.tex_h);
+struct ShadeBwd<JR_SHADER_GOURAUD_TEXTURE> {
+  static JR_DEV void run(const jr_inputs& in, const jr_scene& sc, const jr_grads&,
+                         const float* vary, const float light[3], const float b[3],
+                         const float[3], const float dcol[3],
+                         PixGrad<JR_SHADER_GOURAUD_TEXTURE>& g, float*, int) {
+    wrapped_texel(sc, vary + 9, b, &g.u, &g.v);
     float tex[3];
-    tex_rgb(in.textures, sc.tex_base, sc.tex_h, sc.tex_c, u, t, tex);
-    float dt[3], dl[3];
+    tex_rgb(in.textures, sc.tex_base, sc.tex_h, sc.tex_c, g.u, g.v, tex);
+#pragma unroll
     for (int q = 0; q < 3; ++q) {
-      dt[q] = dcol[q] * light[q];
-      dl[q] = dcol[q] * tex[q];
-    }
-    add_tex(g, sc.tex_base, sc.tex_h, sc.tex_c, u, t, dt);
-    for (int k = 0; k < 3; ++k) {
-      g.db[k] = dot3(dl, v + 3 * k);
-      for (int q = 0; q < 3; ++q) g.dvar[k][q] = b[k] * dl[q];
+      g.tex_g[q] = dcol[q] * light[q];
+      g.dn[q] = dcol[q] * tex[q];
     }
   }
 };
 
 // shaders/phong.py:106-164
 template <>
-struct ShadeBwd<JR_SHADER_PHONG> : CornerBwd<JR_SHADER_PHONG> {
-  // v: the corners' eye-space normals (3 x 3), then their uvs (3 x 2)
-  static JR_DEV void run_v(const jr_inputs& in, const jr_scene& sc, const jr_grads&,
-                           const float* v, const float b[3], const float dcol[3], PixGrad& g,
-                           int) {
-    const float* ne = v;
-    const float* uvv = v + 9;
-    float n[3];
-    for (int q = 0; q < 3; ++q) n[q] = interp(b, ne[q], ne[3 + q], ne[6 + q]);
-    const float uu = interp(b, uvv[0], uvv[2], uvv[4]);
-    const float vv = interp(b, uvv[1], uvv[3], uvv[5]);
-    const int32_t u = floor_mod(f2i_sat(floorf(uu)), sc.tex_w);
-    const int32_t t = floor_mod(f2i_sat(floorf(vv)), sc.tex_h);
-    float tex[3], nn[3], ln[3];
-    tex_rgb(in.textures, sc.tex_base, sc.tex_h, sc.tex_c, u, t, tex);
+struct ShadeBwd<JR_SHADER_PHONG> {
+  static JR_DEV void run(const jr_inputs& in, const jr_scene& sc, const jr_grads&,
+                         const float* vary, const float n[3], const float b[3],
+                         const float ln[3], const float dcol[3],
+                         PixGrad<JR_SHADER_PHONG>& g, float* sg, int) {
+    int32_t u, v;
+    wrapped_texel(sc, vary + 9, b, &u, &v);
+    float tex[3], nn[3];
+    tex_rgb(in.textures, sc.tex_base, sc.tex_h, sc.tex_c, u, v, tex);
     normalise3(n, nn);
-    normalise3(sc.light_direction, ln);
     const float d = dot3(nn, ln);
     float lc[3];
     bool pos = true;
+#pragma unroll
     for (int q = 0; q < 3; ++q) {
       lc[q] = sc.light_colour[q] * d;
       pos = pos && (lc[q] >= 0.0f);
     }
     if (!pos) return;  // the zero branch of the cond carries no gradient
-    float dt[3], dlc[3];
-    float dd = 0.0f;
+    g.u = u;
+    g.v = v;
+    float dd = 0.0f, dnn[3];
+#pragma unroll
     for (int q = 0; q < 3; ++q) {
-      dt[q] = dcol[q] * lc[q];
-      dlc[q] = dcol[q] * tex[q];
-      g.sg[S_LIGHT_COLOUR + q] += dlc[q] * d;
-      dd += dlc[q] * sc.light_colour[q];
+      g.tex_g[q] = dcol[q] * lc[q];
+      const float dlc = dcol[q] * tex[q];
+      sg[S_LIGHT_COLOUR + q] = fmaf(dlc, d, sg[S_LIGHT_COLOUR + q]);
+      dd += dlc * sc.light_colour[q];
     }
-    add_tex(g, sc.tex_base, sc.tex_h, sc.tex_c, u, t, dt);
-    float dnn[3], dln[3], dn[3];
+#pragma unroll
     for (int q = 0; q < 3; ++q) {
       dnn[q] = dd * ln[q];
-      dln[q] = dd * nn[q];
-      g.sg[S_LIGHT_DIR + q] += dln[q];  // normalise's backward applied per tile
+      sg[S_DIR + q] = fmaf(dd, nn[q], sg[S_DIR + q]);  // normalise's backward applied per tile
     }
-    normalise_bwd(n, dnn, dn);
-    for (int k = 0; k < 3; ++k) {
-      g.db[k] = dot3(dn, ne + 3 * k);
-      for (int q = 0; q < 3; ++q) g.dvar[k][q] = b[k] * dn[q];
-    }
+    normalise_bwd(n, dnn, g.dn);
   }
 };
 
-// shaders/phong_darboux.py:116-293: the forward of Shade<PHONG_DARBOUX>
+// shaders/phong_darboux.py:116-293: the forward of Varyings<PHONG_DARBOUX>::pixel
 // with its intermediates, then its reverse.  Beyond phong's terms the
 // gradient reaches the tangent frame: B = [i/|i|, j/|j|, n] with
 // (i, j) = inv(A) @ [du, dv] and A = [t1 - t0; t2 - t0; n] built from the
@@ -263,107 +228,72 @@ struct ShadeBwd<JR_SHADER_PHONG> : CornerBwd<JR_SHADER_PHONG> {
 // positions, uvs and world_to_clip); the normal-map texel gets d(B @ nm).
 template <>
 struct ShadeBwd<JR_SHADER_PHONG_DARBOUX> {
+  using V = Varyings<JR_SHADER_PHONG_DARBOUX>;
   static JR_DEV void run(const jr_inputs& in, const jr_scene& sc, const jr_grads& gr,
-                         const Corner& c, const float b[3], const float dcol[3], PixGrad& g,
-                         int) {
-    float ne[3][3], uvv[3][2];
-    for (int k = 0; k < 3; ++k) {
-      eye_normal(in, sc, c.slot[k], ne[k]);
-      load2(in.uvs, attr_row(in.uv_index, c.slot[k]), uvv[k]);
-    }
-    const int32_t face = in.id_to_face[c.slot[0]];
-    float tri[3][3], tuv[3][2];
-    for (int m = 0; m < 3; ++m) {
-      const int32_t q = in.face_slots[3 * (int64_t)face + m];
-      float h[4];
-      position_clip(in, sc.world_to_clip, q, h);
-      const bool wz = (h[3] == 0.0f);
-      tri[m][0] = wz ? h[0] : h[0] / h[3];
-      tri[m][1] = wz ? h[1] : h[1] / h[3];
-      tri[m][2] = wz ? h[2] : h[2] / h[3];
-      load2(in.uvs, attr_row(in.uv_index, q), tuv[m]);
-    }
-    float n_i[3];
-    for (int q = 0; q < 3; ++q) n_i[q] = interp(b, ne[0][q], ne[1][q], ne[2][q]);
-    const float uu = interp(b, uvv[0][0], uvv[1][0], uvv[2][0]);
-    const float vv = interp(b, uvv[0][1], uvv[1][1], uvv[2][1]);
-    const int32_t u = floor_mod(f2i_sat(floorf(uu)), sc.tex_w);
-    const int32_t v = floor_mod(f2i_sat(floorf(vv)), sc.tex_h);
-    float n[3];
-    normalise3(n_i, n);
-    float A[9], AI[9];
-    for (int q = 0; q < 3; ++q) {
-      A[q] = tri[1][q] - tri[0][q];
-      A[3 + q] = tri[2][q] - tri[0][q];
-      A[6 + q] = n[q];
-    }
-    inv3(A, AI);
-    const float du1 = tuv[1][0] - tuv[0][0], du2 = tuv[2][0] - tuv[0][0];
-    const float dv1 = tuv[1][1] - tuv[0][1], dv2 = tuv[2][1] - tuv[0][1];
-    float iv[3], jv[3];
-    for (int r = 0; r < 3; ++r) {
-      float s = AI[3 * r + 0] * du1;
-      s = s + AI[3 * r + 1] * du2;
-      s = s + AI[3 * r + 2] * 0.0f;
-      iv[r] = s;
-      float t = AI[3 * r + 0] * dv1;
-      t = t + AI[3 * r + 1] * dv2;
-      t = t + AI[3 * r + 2] * 0.0f;
-      jv[r] = t;
-    }
-    float in_[3], jn[3];
-    normalise3(iv, in_);
-    normalise3(jv, jn);
+                         const float* vary, const float n_i[3], const float b[3],
+                         const float ln[3], const float dcol[3],
+                         PixGrad<JR_SHADER_PHONG_DARBOUX>& g, float* sg, int) {
+    int32_t u, v;
+    wrapped_texel(sc, vary + 9, b, &u, &v);
+    float tex[3], nm[3];
+    tex_rgb(in.textures, sc.tex_base, sc.tex_h, sc.tex_c, u, v, tex);
     const int32_t un = index_clamp(u, sc.nmap_w);
     const int32_t vn = index_clamp(v, sc.nmap_h);
-    float nm[3];
     load3(in.normal_maps + sc.nmap_base, un * sc.nmap_h + vn, nm);
+    float n[3], AI[9], iv[3], jv[3], in_[3], jn[3];
+    normalise3(n_i, n);
+    V::tangents(vary, n, AI, iv, jv);
+    normalise3(iv, in_);
+    normalise3(jv, jn);
     float bn[3];
+#pragma unroll
     for (int r = 0; r < 3; ++r) {
       float s = in_[r] * nm[0];
       s = s + jn[r] * nm[1];
       s = s + n[r] * nm[2];
       bn[r] = s;
     }
-    float n2[3], ln[3];
+    float n2[3];
     normalise3(bn, n2);
-    normalise3(sc.light_direction, ln);
     const float d = dot3(n2, ln);
-    float tex[3];
-    tex_rgb(in.textures, sc.tex_base, sc.tex_h, sc.tex_c, u, v, tex);
     float lc[3];
     bool pos = true;
+#pragma unroll
     for (int ch = 0; ch < 3; ++ch) {
       lc[ch] = sc.light_colour[ch] * d;
       pos = pos && (lc[ch] >= 0.0f);
     }
     if (!pos) return;  // the zero branch of the cond carries no gradient
+    g.u = u;
+    g.v = v;
 
     // colour = tex * light_colour * dot(n2, ln)
-    float dt[3], dd = 0.0f;
+    float dd = 0.0f;
+#pragma unroll
     for (int q = 0; q < 3; ++q) {
-      dt[q] = dcol[q] * lc[q];
+      g.tex_g[q] = dcol[q] * lc[q];
       const float dlc = dcol[q] * tex[q];
-      g.sg[S_LIGHT_COLOUR + q] += dlc * d;
+      sg[S_LIGHT_COLOUR + q] = fmaf(dlc, d, sg[S_LIGHT_COLOUR + q]);
       dd += dlc * sc.light_colour[q];
     }
-    add_tex(g, sc.tex_base, sc.tex_h, sc.tex_c, u, v, dt);
-    float dn2[3], dln[3], dbn[3];
+    float dn2[3], dbn[3];
+#pragma unroll
     for (int q = 0; q < 3; ++q) {
       dn2[q] = dd * ln[q];
-      dln[q] = dd * n2[q];
-      g.sg[S_LIGHT_DIR + q] += dln[q];  // normalise's backward applied per tile
+      sg[S_DIR + q] = fmaf(dd, n2[q], sg[S_DIR + q]);  // normalise's backward applied per tile
     }
     normalise_bwd(bn, dn2, dbn);
     // bn = B @ nm with B's columns in_, jn, n
     float din[3], djn[3], dn[3];
+#pragma unroll
     for (int r = 0; r < 3; ++r) {
       din[r] = dbn[r] * nm[0];
       djn[r] = dbn[r] * nm[1];
       dn[r] = dbn[r] * nm[2];
     }
     if (gr.d_normal_maps) {
-      g.nmap_at = sc.nmap_base + 3 * ((int64_t)un * sc.nmap_h + vn);
+      g.us = un;
+      g.vs = vn;
       g.nmap_g[0] = dot3(dbn, in_);
       g.nmap_g[1] = dot3(dbn, jn);
       g.nmap_g[2] = dot3(dbn, n);
@@ -372,8 +302,12 @@ struct ShadeBwd<JR_SHADER_PHONG_DARBOUX> {
     normalise_bwd(iv, din, div);
     normalise_bwd(jv, djn, djv);
     // (i, j) = AI @ (du, dv): dAI = div du^T + djv dv^T, d(du) = AI^T div
+    const float* tuv = vary + V::kTuv;
+    const float du1 = tuv[2] - tuv[0], du2 = tuv[4] - tuv[0];
+    const float dv1 = tuv[3] - tuv[1], dv2 = tuv[5] - tuv[1];
     float dAI[9];
     float ddu1 = 0.0f, ddu2 = 0.0f, ddv1 = 0.0f, ddv2 = 0.0f;
+#pragma unroll
     for (int r = 0; r < 3; ++r) {
       dAI[3 * r + 0] = div[r] * du1 + djv[r] * dv1;
       dAI[3 * r + 1] = div[r] * du2 + djv[r] * dv2;
@@ -383,73 +317,58 @@ struct ShadeBwd<JR_SHADER_PHONG_DARBOUX> {
       ddv1 += djv[r] * AI[3 * r + 0];
       ddv2 += djv[r] * AI[3 * r + 1];
     }
-    g.dtuv[0] = -(ddu1 + ddu2);  // corner 0: u, v
-    g.dtuv[1] = -(ddv1 + ddv2);
-    g.dtuv[2] = ddu1;  // corner 1
-    g.dtuv[3] = ddv1;
-    g.dtuv[4] = ddu2;  // corner 2
-    g.dtuv[5] = ddv2;
+    float* dtuv = g.more + 9;
+    dtuv[0] = -(ddu1 + ddu2);  // corner 0: u, v
+    dtuv[1] = -(ddv1 + ddv2);
+    dtuv[2] = ddu1;  // corner 1
+    dtuv[3] = ddv1;
+    dtuv[4] = ddu2;  // corner 2
+    dtuv[5] = ddv2;
     // dA = -AI^T dAI AI^T
     float T1[9], dA[9];
+#pragma unroll
     for (int p = 0; p < 3; ++p)
+#pragma unroll
       for (int k = 0; k < 3; ++k) {
         float s = 0.0f;
+#pragma unroll
         for (int r = 0; r < 3; ++r) s += AI[3 * r + p] * dAI[3 * r + k];
         T1[3 * p + k] = s;
       }
+#pragma unroll
     for (int p = 0; p < 3; ++p)
+#pragma unroll
       for (int q = 0; q < 3; ++q) {
         float s = 0.0f;
+#pragma unroll
         for (int k = 0; k < 3; ++k) s += T1[3 * p + k] * AI[3 * q + k];
         dA[3 * p + q] = -s;
       }
+#pragma unroll
     for (int q = 0; q < 3; ++q) {
-      g.dtri[0 + q] = -(dA[q] + dA[3 + q]);
-      g.dtri[3 + q] = dA[q];
-      g.dtri[6 + q] = dA[3 + q];
+      g.more[0 + q] = -(dA[q] + dA[3 + q]);
+      g.more[3 + q] = dA[q];
+      g.more[6 + q] = dA[3 + q];
       dn[q] += dA[6 + q];
     }
-    float dni[3];
-    normalise_bwd(n_i, dn, dni);
-    for (int k = 0; k < 3; ++k) {
-      g.db[k] = dot3(dni, ne[k]);
-      for (int q = 0; q < 3; ++q) g.dvar[k][q] = b[k] * dni[q];
-    }
+    normalise_bwd(n_i, dn, g.dn);
   }
 };
 
 // shaders/phong_reflection.py:154-235 and phong_reflection_shadow.py:173-271
-template <bool SHADOW>
+template <int SHADER>
 struct ReflectionBwd {
-  using V = Varyings<SHADOW ? JR_SHADER_PHONG_REFLECTION_SHADOW : JR_SHADER_PHONG_REFLECTION>;
+  static constexpr bool SHADOW = SHADER == JR_SHADER_PHONG_REFLECTION_SHADOW;
+  using V = Varyings<SHADER>;
   static JR_DEV void run(const jr_inputs& in, const jr_scene& sc, const jr_grads& gr,
-                         const Corner& c, const float b[3], const float dcol[3], PixGrad& g,
-                         int scene) {
-    float v[V::N];
-    V::corners(in, sc, c, v);
-    run_v(in, sc, gr, v, b, dcol, g, scene);
-  }
-  // v: the triangle's corner stage (Varyings<>::corners)
-  static JR_DEV void run_v(const jr_inputs& in, const jr_scene& sc, const jr_grads& gr,
-                           const float* vary, const float b[3], const float dcol[3],
-                           PixGrad& g, int scene) {
-    const float* nev = vary;      // eye-space normal of corner k: nev[3k..3k+2]
+                         const float* vary, const float n[3], const float b[3],
+                         const float lh[3], const float dcol[3], PixGrad<SHADER>& g,
+                         float* sg, int scene) {
     const float* uvv = vary + 9;  // uv of corner k: uvv[2k..2k+1]
     const int32_t ti = __float_as_int(vary[V::kTi]);
-    float n[3], uv[2];
-    for (int q = 0; q < 3; ++q) n[q] = interp(b, nev[q], nev[3 + q], nev[6 + q]);
+    float uv[2];
     uv[0] = interp(b, uvv[0], uvv[2], uvv[4]);
     uv[1] = interp(b, uvv[1], uvv[3], uvv[5]);
-    bool lit = true;
-    if (SHADOW) {
-      const float* scd = vary + 15;  // homogeneous-normalised shadow clip of corner k
-      float s4[4], sv[4];
-      for (int q = 0; q < 4; ++q) s4[q] = interp(b, scd[q], scd[4 + q], scd[8 + q]);
-      apply4(sc.shadow_viewport, s4[0], s4[1], s4[2], s4[3], sv);
-      const float* map = in.shadow_maps + (int64_t)scene * in.shadow_w * in.shadow_h;
-      lit = (sv[2] / sv[3]) <= shadow_get(map, in.shadow_w, in.shadow_h, sv[0] / sv[3],
-                                          sv[1] / sv[3]);
-    }
     // forward of reflection_terms with its intermediates
     const int32_t s0 = __float_as_int(vary[V::kShape]), s1 = __float_as_int(vary[V::kShape + 1]);
     float f0 = modf_frac(uv[0]), f1 = modf_frac(uv[1]);
@@ -458,15 +377,26 @@ struct ReflectionBwd {
     const int32_t shift = (int32_t)((uint32_t)ti * (uint32_t)sc.tex_offset);
     const int32_t u0 = f2i_sat(floorf(f0 * (float)s0 + (float)shift));
     const int32_t v0 = f2i_sat(floorf(f1 * (float)s1));
-    const int32_t u = index_clamp(u0, sc.tex_w), v = index_clamp(v0, sc.tex_h);
-    const int32_t us = index_clamp(u0, sc.spec_w), vs = index_clamp(v0, sc.spec_h);
-    float tex[3];
-    tex_rgb(in.textures, sc.tex_base, sc.tex_h, sc.tex_c, u, v, tex);
-    const int64_t spec_at = sc.spec_base + (int64_t)us * sc.spec_h + vs;
-    const float S = in.specular_maps[spec_at];
-    float nh[3], lh[3];
+    g.u = index_clamp(u0, sc.tex_w);
+    g.v = index_clamp(v0, sc.tex_h);
+    g.us = index_clamp(u0, sc.spec_w);
+    g.vs = index_clamp(v0, sc.spec_h);
+    // the three lookups are issued together
+    float tex[3], depth = 0.0f, sz = 0.0f;
+    tex_rgb(in.textures, sc.tex_base, sc.tex_h, sc.tex_c, g.u, g.v, tex);
+    const float S = in.specular_maps[sc.spec_base + (int64_t)g.us * sc.spec_h + g.vs];
+    if (SHADOW) {
+      const float* scd = vary + 15;  // homogeneous-normalised shadow clip of corner k
+      float s4[4], sv[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) s4[q] = interp(b, scd[q], scd[4 + q], scd[8 + q]);
+      apply4(sc.shadow_viewport, s4[0], s4[1], s4[2], s4[3], sv);
+      sz = sv[2] / sv[3];
+      const float* map = in.shadow_maps + (int64_t)scene * in.shadow_w * in.shadow_h;
+      depth = shadow_get(map, in.shadow_w, in.shadow_h, sv[0] / sv[3], sv[1] / sv[3]);
+    }
+    float nh[3];
     normalise3(n, nh);
-    normalise3(sc.light_dir_eye, lh);
     const float d = dot3(nh, lh);
     const float diff = max_nan(d, 0.0f);
     const float two_d = 2.0f * d;
@@ -474,66 +404,58 @@ struct ReflectionBwd {
     float rh[3];
     normalise3(qv, rh);
     const float m = max_nan(rh[2], 0.0f);
-    // the forward's power (pow_unit: within 3e-7 of powf for m in [0, 1])
+    // the forward's power (pow_unit: within 3e-7 of powf for m in [0, 1]) and the
+    // one of its derivative
     const float spec = pow_unit(m, S);
+    const float slope = S == 0.0f ? 0.0f : S * pow_unit(m, S - 1.0f);
+    const bool lit = !SHADOW || sz <= depth;
 
-    float dt[3], ddiff = 0.0f, dspec = 0.0f;
+    float ddiff = 0.0f, dspec = 0.0f;
+#pragma unroll
     for (int q = 0; q < 3; ++q) {
       const float k = sc.diffuse[q] * diff + sc.specular[q] * spec;
       const float sh = lit ? 1.0f : 1.0f - sc.shadow_strength[q];
-      g.sg[S_AMBIENT + q] += dcol[q] * tex[q];
-      float dk;
-      if (SHADOW) {
-        dt[q] = dcol[q] * (sc.ambient[q] + (sh * k) * sc.light_colour[q]);
-        dk = dcol[q] * sh * tex[q] * sc.light_colour[q];
-        g.sg[S_LIGHT_COLOUR + q] += dcol[q] * (sh * k) * tex[q];
-        if (!lit) g.sg[S_STRENGTH + q] += -dcol[q] * k * tex[q] * sc.light_colour[q];
-      } else {
-        dt[q] = dcol[q] * (sc.ambient[q] + k * sc.light_colour[q]);
-        dk = dcol[q] * sc.light_colour[q] * tex[q];
-        g.sg[S_LIGHT_COLOUR + q] += dcol[q] * k * tex[q];
-      }
-      g.sg[S_DIFFUSE + q] += dk * diff;
-      g.sg[S_SPECULAR + q] += dk * spec;
+      const float ct = dcol[q] * tex[q];
+      const float cs = SHADOW ? sh * ct : ct;
+      const float dk = SHADOW ? dcol[q] * sh * tex[q] * sc.light_colour[q]
+                              : dcol[q] * sc.light_colour[q] * tex[q];
+      g.tex_g[q] = dcol[q] * (sc.ambient[q] + (SHADOW ? sh * k : k) * sc.light_colour[q]);
+      sg[S_AMBIENT + q] += ct;
+      if constexpr (SHADOW)
+        sg[S_STRENGTH + q] =
+            lit ? sg[S_STRENGTH + q]
+                : fmaf(-k, ct * sc.light_colour[q], sg[S_STRENGTH + q]);
+      sg[S_DIFFUSE + q] = fmaf(cs, diff, sg[S_DIFFUSE + q]);
+      sg[S_SPECULAR + q] = fmaf(cs, spec, sg[S_SPECULAR + q]);
       ddiff += dk * sc.diffuse[q];
       dspec += dk * sc.specular[q];
     }
-    add_tex(g, sc.tex_base, sc.tex_h, sc.tex_c, u, v, dt);
-    if (gr.d_specular_maps) {
-      const float lg = logf(m == 0.0f ? 1.0f : m);
-      g.spec_at = spec_at;
-      g.spec_g = dspec * lg * spec;
-    }
-    const float dm = dspec * (S == 0.0f ? 0.0f : S * pow_unit(m, S - 1.0f));
+    if (gr.d_specular_maps)
+      g.spec_g = dspec * logf(m == 0.0f ? 1.0f : m) * spec;
+    else
+      g.us = -1;
+    const float dm = dspec * slope;
     const float dr[3] = {0.0f, 0.0f, dm * max_grad(rh[2], 0.0f)};
     float dq[3];
     normalise_bwd(qv, dr, dq);
-    float dnh[3], dlh[3];
-    float dtwo_d = dot3(dq, nh);
-    for (int q = 0; q < 3; ++q) {
-      dnh[q] = two_d * dq[q];
-      dlh[q] = -dq[q];
-    }
+    const float dtwo_d = dot3(dq, nh);
     const float dd = 2.0f * dtwo_d + ddiff * max_grad(d, 0.0f);
+    float dnh[3];
+#pragma unroll
     for (int q = 0; q < 3; ++q) {
-      dnh[q] += dd * lh[q];
-      dlh[q] += dd * nh[q];
+      dnh[q] = two_d * dq[q] + dd * lh[q];
+      // normalise's backward is linear in its cotangent: applied once per tile
+      sg[S_DIR + q] += fmaf(dd, nh[q], -dq[q]);
     }
-    float dn[3];
-    normalise_bwd(n, dnh, dn);
-    // normalise's backward is linear in its cotangent: applied once per tile
-    for (int q = 0; q < 3; ++q) g.sg[S_LIGHT_DIR_EYE + q] += dlh[q];
-    for (int k = 0; k < 3; ++k) {
-      g.db[k] = dot3(dn, nev + 3 * k);
-      for (int q = 0; q < 3; ++q) g.dvar[k][q] = b[k] * dn[q];
-    }
+    normalise_bwd(n, dnh, g.dn);
   }
 };
 
 template <>
-struct ShadeBwd<JR_SHADER_PHONG_REFLECTION> : ReflectionBwd<false> {};
+struct ShadeBwd<JR_SHADER_PHONG_REFLECTION> : ReflectionBwd<JR_SHADER_PHONG_REFLECTION> {};
 template <>
-struct ShadeBwd<JR_SHADER_PHONG_REFLECTION_SHADOW> : ReflectionBwd<true> {};
+struct ShadeBwd<JR_SHADER_PHONG_REFLECTION_SHADOW>
+    : ReflectionBwd<JR_SHADER_PHONG_REFLECTION_SHADOW> {};
 
 // v moved across lanes by the DPP pattern CTRL (lanes without a source get 0).
 template <int CTRL>
@@ -541,95 +463,90 @@ JR_DEV float dpp_move(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
 }
 
-// Sum over the 64 lanes of the wavefront, returned to every lane: lane pairs
-// and quads (quad_perm [1,0,3,2], [2,3,0,1]), rows of 16 (row_ror 4, 8), then
-// rows 0-1 into 1 and 2-3 into 3 (row_bcast 15) and rows 0-1 into 2-3
-// (row_bcast 31), so lane 63 holds the total; all register-to-register, no
-// LDS.  Call with every lane active.
-JR_DEV float wave_sum(float v) {
-  v += dpp_move<0xb1>(v);
-  v += dpp_move<0x4e>(v);
-  v += dpp_move<0x124>(v);
-  v += dpp_move<0x128>(v);
-  v += dpp_move<0x142>(v);
-  v += dpp_move<0x143>(v);
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
-}
-
-// d[at + c] += v[c] (c < n), summed first in an LDS table of (index, sum)
-// entries shared by the tile's pixels, so a texel that several pixels read
-// costs one global atomic per channel and tile; indices beyond the table's
-// capacity (or beyond 2^31) are added directly.
-// Sums a lane could not stage (its table full), kept in registers (at most
-// KMAX, later ones add at once) and added to global memory after the pixel
-// loop, so that no global atomic sits between the loop's loads (a
-// wavefront's memory operations complete in order, so a later load would
-// wait for the atomic's round trip).  A 16x16 tile whose 256 pixels read 256
-// distinct texels fills a 128-entry table after two of a lane's four pixels,
-// which leaves two per lane.
-template <int NC, int KMAX>
-struct Pending {
-  int64_t at[KMAX];
-  float v[KMAX][NC];
-  JR_DEV Pending() {
+// The totals over the 64 lanes of the wavefront of N <= 32 values a lane: lane l
+// returns that of value l / 2 (l / 2 < N).  A step of the reduction halves the
+// lanes that share a value and the values that a lane holds: in step 16 the
+// lower half of the wavefront goes on with values 0..15 and the upper half with
+// 16..31, and so on, so 32 values take 16 + 8 + 4 + 2 + 1 + 1 additions, where one
+// value at a time takes six each, and their totals are added to memory by one
+// instruction.  Call with every lane active.
+template <int N>
+JR_DEV float wave_totals(const float (&v)[N]) {
+  static_assert(N <= 32, "one value per lane pair");
+  float a[N];
 #pragma unroll
-    for (int k = 0; k < KMAX; ++k) at[k] = -1;
-  }
-  // false when every register entry is taken
-  JR_DEV bool push(int64_t a, int32_t n, const float* g) {
+  for (int i = 0; i < N; ++i) a[i] = v[i];
+  const int lane = threadIdx.x & 63;
+  int n = N;
 #pragma unroll
-    for (int k = 0; k < KMAX; ++k) {
-      if (at[k] < 0) {
-        at[k] = a;
+  for (int half = 16; half >= 1; half >>= 1) {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) v[k][c] = c < n ? g[c] : 0.0f;
-        return true;
+    for (int i = 0; i < half && i < n; ++i) {
+      const bool pair = i + half < n;
+      const float x = a[i], y = pair ? a[i + half] : x;
+      if (half >= 8) {
+        const auto r = half == 16
+                           ? __builtin_amdgcn_permlane32_swap(__float_as_uint(x),
+                                                              __float_as_uint(y), false, false)
+                           : __builtin_amdgcn_permlane16_swap(__float_as_uint(x),
+                                                              __float_as_uint(y), false, false);
+        a[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+      } else {
+        const bool up = (lane & (2 * half)) != 0;
+        const float keep = up ? y : x, give = up ? x : y;
+        a[i] = keep + (half == 4   ? dpp_move<0x128>(give)    // row_ror:8
+                       : half == 2 ? dpp_move<0x141>(give)    // row_half_mirror
+                                   : dpp_move<0x4e>(give));   // quad_perm [2,3,0,1]
       }
     }
-    return false;
+    n = n < half ? n : half;
   }
-  JR_DEV void flush(float* __restrict__ d) {
-#pragma unroll
-    for (int k = 0; k < KMAX; ++k)
-      if (at[k] >= 0)
-#pragma unroll
-        for (int c = 0; c < NC; ++c)
-          if (v[k][c] != 0.0f) atomicAdd(d + at[k] + c, v[k][c]);
-  }
-};
+  return a[0] + dpp_move<0xb1>(a[0]);  // quad_perm [1,0,3,2]
+}
 
+// Sums per map entry in LDS: NC floats for each of up to CAP distinct keys, so
+// that an entry which several pixels of the wavefront read costs one global
+// atomic per channel.  What finds no place near its own is added to memory at
+// once; its acknowledgement then holds up the loads issued after it (a wavefront's
+// memory operations complete in order), so the table is as large as the number of
+// pixels where nearly every pixel has its own entry.
 constexpr int32_t kStageProbes = 16;
 
-template <int CAP, int NC, int KMAX>
-JR_DEV void stage_add(int32_t* tab, float (*val)[NC], float* __restrict__ d, int64_t at,
-                      int32_t n, const float* v, Pending<NC, KMAX>& pend) {
-  if (!d || at < 0) return;
-  // a texel table fills up where nearly every pixel reads its own texel: a
-  // miss then costs kStageProbes LDS operations, not CAP
-  const int32_t e = at < 0x7FFFFFFFLL ? table_insert(tab, CAP, (int32_t)at, kStageProbes) : -1;
-  if (e < 0) {
-    if (!pend.push(at, n, v))
-      for (int c = 0; c < n; ++c)
-        if (v[c] != 0.0f) atomicAdd(d + at + c, v[c]);
-    return;
-  }
-  for (int c = 0; c < n; ++c)
-    if (v[c] != 0.0f) atomicAdd(&val[e][c], v[c]);
-}
-
-// Adds the staged sums to d (n channels per entry) and leaves the table free.
-// Lanes take consecutive (entry, channel) pairs, so the channels of one entry
-// are added by neighbouring lanes of one instruction (same cache line).
 template <int CAP, int NC>
-JR_DEV void flush_adds(int32_t* tab, float (*val)[NC], float* __restrict__ d, int32_t n) {
-  if (!d) return;
-  for (int idx = threadIdx.x; idx < CAP * n; idx += blockDim.x) {
-    const int e = n == 3 ? idx / 3 : (n == 1 ? idx : idx / n);
-    const int c = idx - e * n;
-    const int32_t at = tab[e];
-    if (at >= 0 && val[e][c] != 0.0f) atomicAdd(d + at + c, val[e][c]);
+struct SumTable {
+  int32_t key[CAP];
+  float v[NC][CAP];
+  JR_DEV void clear() {
+    for (int e = threadIdx.x; e < CAP; e += 64) {
+      key[e] = -1;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) v[c][e] = 0.0f;
+    }
   }
-}
+  // g to entry k; to_memory(k, c, x): x to channel c of an entry in memory
+  template <class Add>
+  JR_DEV void add(int32_t k, const float* g, Add to_memory) {
+    const int32_t e = table_insert(key, CAP, k, kStageProbes);
+    if (e >= 0) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) atomicAdd(&v[c][e], g[c]);
+    } else {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) to_memory(k, c, g[c]);
+    }
+  }
+  // Adds the sums to memory.  Lanes take consecutive (entry, channel) pairs, so
+  // the channels of one entry are added by neighbouring lanes of one instruction
+  // (same cache line).
+  template <class Add>
+  JR_DEV void flush(Add to_memory) {
+    for (int idx = threadIdx.x; idx < CAP * NC; idx += 64) {
+      const int e = idx / NC, c = idx - NC * e;
+      const int32_t k = key[e];
+      if (k != -1) to_memory(k, c, v[c][e]);
+    }
+  }
+};
 
 struct BwdArgs {
   jr_inputs in;
@@ -662,6 +579,14 @@ struct BwdArgs {
 constexpr int kHdrMagicLo = 0, kHdrMagicHi = 1, kHdrTris = 2, kHdrFill = 3, kHdrAcc = 4;
 constexpr uint32_t kMagicLo = 0x6a724277u, kMagicHi = 0x73706b31u;
 
+// The calling kernel's first argument, of type T, in the kernel argument segment.
+template <class T>
+using KernArgs = const __attribute__((address_space(4))) T*;
+template <class T>
+JR_DEV KernArgs<T> kernel_args() {
+  return (KernArgs<T>)__builtin_amdgcn_kernarg_segment_ptr();
+}
+
 // A scene's pixels in 2x2 blocks, one wavefront per 64 consecutive blocks of
 // this enumeration: the full tiles of 8 x 8 blocks (16 x 16 pixels) first,
 // tile by tile, so that each is one wavefront with lane l owning the block
@@ -669,334 +594,460 @@ constexpr uint32_t kMagicLo = 0x6a724277u, kMagicHi = 0x73706b31u;
 // row) and those right of them (rw per column), which share wavefronts
 // instead of leaving most lanes of a partial tile idle (an 84 x 84 frame
 // takes 28 wavefronts, not 36).  Where that saves few wavefronts every tile,
-// partial ones included, is a wavefront of its own.  The wavefront's
-// distinct primitives (up to kBwdCap) get their setup (M^-1 columns and clip
-// z) and, for the split shaders, their corner stage computed once, by one
-// lane each, into LDS.  A lane sums the cotangents of consecutive pixels of
-// one triangle (and the gradients of consecutive pixels on one texel) in
-// registers and adds a run to the LDS sums only when it ends, so neighbouring
-// pixels, which mostly share both, cost one LDS atomic instead of four; the
-// LDS sums reach the global accumulators once per (wavefront, triangle) and
-// per (wavefront, texel).  Pixels of primitives beyond the table's capacity compute
-// their own and add directly.
-constexpr int kBwdCap = 32;
-constexpr int kTexCap = 128;  // distinct texels summed in LDS per wavefront
-constexpr int kSpecCap = 64;  // distinct specular-map entries
+// partial ones included, is a wavefront of its own.
+//
+// A wavefront works in rounds of up to tri_cap() distinct triangles (mostly one):
+// their setup and corner stage, by one lane per triangle and per corner, go to
+// LDS; then each lane goes over its four pixels.  A lane sums consecutive pixels of
+// one triangle, and of one texel, in registers and adds a run to the LDS sums when
+// it ends, so neighbouring pixels, which mostly share both, cost one LDS atomic
+// instead of four; the LDS sums reach memory once per (wavefront, triangle) and
+// (wavefront, map entry).
+//
+// What bounds it: the LDS and round trips to memory.  The LDS takes a turn for
+// each lane of an atomic on one address, and half of a 480x270 frame's wavefronts
+// see one or two large triangles: 512 of them spent 2,470 LDS cycles per wavefront
+// beside 700 cycles' worth of VALU issue.  With the lanes' last runs summed across
+// the wavefront (1,320 LDS cycles), a fourth wavefront per SIMD (162 registers ->
+// 128: scalars read again for each pixel instead of spilt into vector registers,
+// no own path for triangles beyond the table) and the scene's sums reduced
+// together, k_bwd_pixels went from 2,972 to 2,238 us on those 512 frames and the
+// step from 5,205 to 4,465 us; 23 views of 201x187 216 -> 202 us.
+// 16 workgroups' LDS on a CU, 4 wavefronts per SIMD as 128 registers allow, takes
+// at most 10 KiB each.
+constexpr int tri_cap(int shader) {
+  return shader == JR_SHADER_PHONG_REFLECTION_SHADOW || shader == JR_SHADER_PHONG_DARBOUX ? 28
+                                                                                         : 32;
+}
+// distinct texels summed in LDS: the reflection shaders' maps repeat over a merged
+// scene's objects, the others' have about a texel per pixel
+constexpr int tex_cap(int shader) { return reflects(shader) ? 128 : 224; }
+// Lanes on one triangle (texel) from which a sum across the wavefront (some 95
+// instructions for 18 sums, 40 for 4) replaces their LDS atomics, and how many
+// triangles (texels) are looked at.
+constexpr int kShared = 8, kSearched = 8;
+constexpr int kTexShared = 16, kTexSearched = 4;
+constexpr int kMapCap = 32;  // entries of a second map (normal map, specular map)
 
-template <int SHADER>
-__global__ __launch_bounds__(64) void k_bwd_pixels(BwdArgs a) {
-  constexpr int NV = Varyings<SHADER>::N;
+template <int SHADER, bool DZ>
+__global__ __launch_bounds__(64)
+__attribute__((amdgpu_waves_per_eu(SHADER == JR_SHADER_PHONG_DARBOUX ? 2 : 4, 8))) void k_bwd_pixels(BwdArgs) {
+  using V = Varyings<SHADER>;
+  constexpr int NV = V::N;
   constexpr int NS = (12 + NV) | 1;  // record stride (odd: no LDS bank conflicts)
-  __shared__ float trec[kBwdCap * NS];
+  constexpr int CAP = tri_cap(SHADER);
   constexpr int ACC = AccOf<SHADER>::N;
+  // a triangle's sums in a lane and in LDS: its accumulators without A_Z where no
+  // depth gradient comes in (DZ)
+  constexpr int NR = DZ ? ACC : ACC - 3;
+  constexpr int R_VAR = 9, R_Z = 18, R_TRI = DZ ? 21 : 18;
+  constexpr int AS = NR | 1;  // odd row stride: lanes of different rows hit different banks
   constexpr bool DARBOUX = SHADER == JR_SHADER_PHONG_DARBOUX;
-  constexpr int kNmapCap = DARBOUX ? kTexCap : 1;  // distinct normal-map texels
-  constexpr int AS = ACC | 1;  // odd row stride: lanes of different rows hit different banks
-  __shared__ float acc[kBwdCap][AS];
-  __shared__ int32_t tab[kBwdCap];
-  __shared__ int32_t tex_tab[kTexCap];
-  __shared__ float tex_val[kTexCap][3];
-  __shared__ int32_t spec_tab[kSpecCap];
-  __shared__ float spec_val[kSpecCap][1];
-  __shared__ int32_t nmap_tab[kNmapCap];
-  __shared__ float nmap_val[kNmapCap][3];
+  constexpr bool REFLECT = reflects(SHADER);
+  constexpr int NT = REFLECT ? 4 : 3;  // a texel's channels, and its specular exponent's
+  constexpr int N2 = DARBOUX ? 3 : 1;
+  __shared__ float trec[CAP * NS];
+  __shared__ float acc[CAP][AS];
+  __shared__ int32_t tab[CAP];
+  __shared__ float light[3];
+  __shared__ SumTable<(NV > 9 ? tex_cap(SHADER) : 1), NT> tex_tab;
+  __shared__ SumTable<DARBOUX || REFLECT ? kMapCap : 1, N2> map_tab;
+  // The kernel's arguments and the scene's values are read where they are used
+  // (scalar loads): kept over the whole kernel, with what is computed from them,
+  // they take three times the scalar registers there are, and what has no place is
+  // moved through vector registers lane by lane.  read_again() makes the compiler
+  // forget the values it has.
+  KernArgs<BwdArgs> ap = kernel_args<BwdArgs>();
+  const jr_scene* sp = nullptr;
+  auto read_again = [&]() { asm volatile("" : "+s"(ap), "+s"(sp)); };
+  auto args = [&]() -> const BwdArgs& { return *(const BwdArgs*)ap; };
+  auto scene = [&]() -> const jr_scene& { return *sp; };
   const int lane = threadIdx.x;
   const int32_t gt = (int32_t)blockIdx.x;
-  const int32_t s = udiv31(gt, a.T_m, a.T_sh);
+  const int32_t s = udiv31(gt, args().T_m, args().T_sh);
   // the first pixel (bi, bj) of the lane's block, number Q of the scene's blocks
-  const int32_t Q = 64 * (gt - s * a.T) + lane;
+  const int32_t Q = 64 * (gt - s * args().T) + lane;
   int32_t bi, bj;
-  if (Q < a.full_end) {  // a full tile per wavefront, its blocks row by row
+  if (Q < args().full_end) {  // a full tile per wavefront, its blocks row by row
     const int32_t tile = Q >> 6;
-    const int32_t tx = udiv31(tile, a.fy_m, a.fy_sh), ty = tile - tx * a.FY;
+    const int32_t tx = udiv31(tile, args().fy_m, args().fy_sh), ty = tile - tx * args().FY;
     bi = 16 * tx + 2 * ((Q >> 3) & 7);
     bj = 16 * ty + 2 * (Q & 7);
-  } else if (Q < a.bottom_end) {  // below the full tiles, rh blocks per row
-    const int32_t q = Q - a.full_end;
-    const int32_t row = udiv31(q, a.rh_m, a.rh_sh);
+  } else if (Q < args().bottom_end) {  // below the full tiles, rh blocks per row
+    const int32_t q = Q - args().full_end;
+    const int32_t row = udiv31(q, args().rh_m, args().rh_sh);
     bi = 2 * row;
-    bj = 16 * a.FY + 2 * (q - row * a.rh);
+    bj = 16 * args().FY + 2 * (q - row * args().rh);
   } else {  // right of them over the whole height, rw blocks per column
-    const int32_t q = Q - a.bottom_end;
-    const int32_t col = udiv31(q, a.rw_m, a.rw_sh);
-    bi = 16 * a.FX + 2 * (q - col * a.rw);
+    const int32_t q = Q - args().bottom_end;
+    const int32_t col = udiv31(q, args().rw_m, args().rw_sh);
+    bi = 16 * args().FX + 2 * (q - col * args().rw);
     bj = 2 * col;
   }
-  if (Q >= a.nq) bi = a.W;  // past the scene's blocks: no pixels
-  const jr_scene& sc = a.scenes[s];
-  const float* vp = sc.viewport;
-  // reciprocals for the viewport gradients only (x and y themselves are the
-  // forward's quotients)
-  const float ivp0 = 1.0f / vp[0], ivp5 = 1.0f / vp[5];
-  auto pixel_of = [&](int q, int32_t* i_out, int32_t* j_out) -> int32_t {
-    const int32_t i = bi + (q >> 1);
-    const int32_t j = bj + (q & 1);
-    *i_out = i;
-    *j_out = j;
-    if (i >= a.W || j >= a.H) return -1;
-    const int32_t t = a.prim_id[(int64_t)s * a.W * a.H + (int64_t)i * a.H + j];
-    return t < a.in.n_tris ? t : -1;
-  };
+  sp = args().scenes + s;
+  const int64_t pix0 = (int64_t)s * args().W * args().H + (int64_t)bi * args().H + bj;
+  // the block's pixels, q = 2 (i - bi) + (j - bj), that are in the picture
+  uint32_t todo = 0u;
+  if (Q < args().nq && bi < args().W && bj < args().H)
+    todo = 1u | (bj + 1 < args().H ? 2u : 0u) | (bi + 1 < args().W ? 4u : 0u) |
+           (bi + 1 < args().W && bj + 1 < args().H ? 8u : 0u);
+  const float* vp = scene().viewport;
+  const float x0 = pix_x(bi, vp), x1 = pix_x(bi + 1, vp);
+  const float y0 = pix_y(bj, vp), y1 = pix_y(bj + 1, vp);
 
-  // the tile's distinct primitives; the texel and specular-map sum tables
-  if (lane < kBwdCap) tab[lane] = -1;
-  for (int e = lane; e < kTexCap; e += 64) {
-    tex_tab[e] = -1;
-    tex_val[e][0] = tex_val[e][1] = tex_val[e][2] = 0.0f;
+  // sums per map entry.  A texel's specular exponent has the texel's number where
+  // the two maps have one shape (uniform): then its gradient is the texel's
+  // fourth channel.  A map of 2^32 texels and more is added to directly.
+  const bool huge = (int64_t)scene().tex_w * scene().tex_h >= 0xFFFFFFFFLL ||
+                    (REFLECT && (int64_t)scene().spec_w * scene().spec_h >= 0xFFFFFFFFLL) ||
+                    (DARBOUX && (int64_t)scene().nmap_w * scene().nmap_h >= 0xFFFFFFFFLL);
+  const bool one_map = REFLECT && args().gr.d_textures && args().gr.d_specular_maps &&
+                       scene().tex_w == scene().spec_w && scene().tex_h == scene().spec_h;
+  auto texel_at = [&](int64_t m, int c, float x) {
+    if (x == 0.0f) return;
+    if (REFLECT && c == 3)
+      atomicAdd(args().gr.d_specular_maps + scene().spec_base + m, x);
+    else if (c < scene().tex_c)
+      atomicAdd(args().gr.d_textures + scene().tex_base + m * scene().tex_c + c, x);
+  };
+  auto entry_at = [&](int64_t m, int c, float x) {
+    if (x == 0.0f) return;
+    if (REFLECT) atomicAdd(args().gr.d_specular_maps + scene().spec_base + m, x);
+    if (DARBOUX) atomicAdd(args().gr.d_normal_maps + scene().nmap_base + 3 * m + c, x);
+  };
+  auto add_texel = [&](int32_t key, int c, float x) { texel_at((uint32_t)key, c, x); };
+  auto add_entry = [&](int32_t key, int c, float x) { entry_at((uint32_t)key, c, x); };
+  if (lane == 0) {
+    float l[3] = {0.0f, 0.0f, 0.0f};
+    if constexpr (NV > 0) V::scene_terms(scene(), l);
+    light[0] = l[0];
+    light[1] = l[1];
+    light[2] = l[2];
   }
-  for (int e = lane; e < kSpecCap; e += 64) {
-    spec_tab[e] = -1;
-    spec_val[e][0] = 0.0f;
-  }
-  for (int e = lane; e < kNmapCap; e += 64) {
-    nmap_tab[e] = -1;
-    nmap_val[e][0] = nmap_val[e][1] = nmap_val[e][2] = 0.0f;
-  }
-  __syncthreads();
+  tex_tab.clear();
+  if constexpr (REFLECT || DARBOUX) map_tab.clear();
+  int32_t tex_key = -1;  // the lane's open run of pixels on one texel
+  float tex_sum[NT];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    int32_t i, j;
-    const int32_t t = pixel_of(q, &i, &j);
-    if (t >= 0) (void)table_insert(tab, kBwdCap, t);
-  }
-  __syncthreads();
-  if (lane < kBwdCap) {
-    for (int k = 0; k < ACC; ++k) acc[lane][k] = 0.0f;
-    const int32_t t = tab[lane];
-    if (t >= 0) {
-      TriSetup ts;
-      tri_setup(a.in, sc, t, ts);
-      float* r = trec + lane * NS;
-      for (int k = 0; k < 3; ++k) {
-        const float4 c = rec_col(ts, k);
-        r[4 * k + 0] = c.x;
-        r[4 * k + 1] = c.y;
-        r[4 * k + 2] = c.z;
-        r[4 * k + 3] = c.w;
-      }
-    }
-  }
-  // the corner stage: one lane per corner of each listed triangle
-  if constexpr (NV > 0) {
-    for (int idx = lane; idx < 3 * kBwdCap; idx += 64) {
-      const int e = idx / 3, k = idx - 3 * e;
-      const int32_t t = tab[e];
-      if (t >= 0) Varyings<SHADER>::corner(a.in, sc, corner_slots(a.in, t), k, trec + e * NS + 12);
-    }
-  }
-  __syncthreads();
+  for (int c = 0; c < NT; ++c) tex_sum[c] = 0.0f;
 
-  PixGrad g;
-  for (int q = 0; q < S_COUNT; ++q) g.sg[q] = 0.0f;
-  // the lane's open runs: triangle (its table entry, or -1 beyond the table),
-  // texel and specular-map entry, with their sums
-  int32_t run_t = -1, run_slot = -1;
-  float run_v[ACC];
-  for (int k = 0; k < ACC; ++k) run_v[k] = 0.0f;
-  int64_t run_tex = -1, run_spec = -1;
-  int32_t run_tex_n = 0;
-  float run_tex_g[3] = {0.0f, 0.0f, 0.0f}, run_spec_g = 0.0f;
-  int64_t run_nmap = -1;
-  float run_nmap_g[3] = {0.0f, 0.0f, 0.0f};
-  Pending<3, 2> pend_tex;
-  Pending<1, 1> pend_spec;
-  Pending<3, 2> pend_nmap;
-  auto flush_tri = [&]() {
-    if (run_t < 0) return;
-    if (run_slot >= 0) {
-      for (int k = 0; k < ACC; ++k)
-        if (run_v[k] != 0.0f) atomicAdd(&acc[run_slot][k], run_v[k]);
-    } else {
-      a.touched[run_t] = s + 1;  // k_bwd_tris only visits touched triangles
-      for (int k = 0; k < ACC; ++k)
-        if (run_v[k] != 0.0f) atomicAdd(a.tacc + (int64_t)run_t * ACC + k, run_v[k]);
+  // the shader's sums, then the viewport's entries 10 and 11 (DZ)
+  constexpr int NSH = scene_sums(SHADER), NSG = NSH + (DZ ? 2 : 0);
+  float sg[NSG > 0 ? NSG : 1];
+#pragma unroll
+  for (int q = 0; q < NSG; ++q) sg[q] = 0.0f;
+
+  while (__ballot(todo != 0u) != 0) {
+    read_again();
+    // the round's distinct triangles
+    if (lane < CAP) tab[lane] = -1;
+    for (int k = lane; k < CAP * AS; k += 64) (&acc[0][0])[k] = 0.0f;
+    __syncthreads();
+    int32_t t4[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      t4[q] = (todo >> q) & 1u ? args().prim_id[pix0 + (q >> 1) * args().H + (q & 1)] : -1;
+    uint32_t slots = 0u;  // per pixel its triangle's table entry, 255: not in this round
+    int32_t last = -1, last_e = 255;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int32_t t = t4[q] < args().in.n_tris ? t4[q] : -1;
+      if (t < 0) {
+        todo &= ~(1u << q);  // background
+        slots |= 255u << (8 * q);
+        continue;
+      }
+      if (t != last) {
+        last = t;
+        last_e = table_insert(tab, CAP, t) & 255;
+      }
+      slots |= (uint32_t)last_e << (8 * q);
+      if (last_e != 255) todo &= ~(1u << q);
     }
-    for (int k = 0; k < ACC; ++k) run_v[k] = 0.0f;
-  };
-#pragma unroll 1
-  for (int q = 0; q < 4; ++q) {
-    int32_t i, j;
-    const int32_t t = pixel_of(q, &i, &j);
-    if (t != run_t) {
-      flush_tri();
-      run_t = t;
-      run_slot = t >= 0 ? table_insert(tab, kBwdCap, t) : -1;  // finds its entry
-    }
-    const int32_t e_slot = run_slot;
-    const int64_t pix = (int64_t)s * a.W * a.H + (int64_t)i * a.H + j;
-    g.tex_at = -1;
-    g.spec_at = -1;
-    g.nmap_at = -1;
-    if constexpr (DARBOUX) {
-      for (int k = 0; k < 9; ++k) g.dtri[k] = 0.0f;
-      for (int k = 0; k < 6; ++k) g.dtuv[k] = 0.0f;
-    }
-    g.tex_n = 0;
-    g.spec_g = 0.0f;
-    for (int k = 0; k < 3; ++k) g.tex_g[k] = 0.0f;
-    float vals[ACC];
-    for (int k = 0; k < ACC; ++k) vals[k] = 0.0f;
-    if (t >= 0) {
-      float4 r0, r1, r2;
-      float v[NV > 0 ? NV : 1];
-      if (e_slot >= 0) {
-        const float* r = trec + e_slot * NS;
-        r0 = make_float4(r[0], r[1], r[2], r[3]);
-        r1 = make_float4(r[4], r[5], r[6], r[7]);
-        r2 = make_float4(r[8], r[9], r[10], r[11]);
-        if constexpr (NV > 0)
-          for (int k = 0; k < NV; ++k) v[k] = r[12 + k];
-      } else {
+    __syncthreads();
+    if (lane < CAP) {
+      const int32_t t = tab[lane];
+      if (t >= 0) {
         TriSetup ts;
-        tri_setup(a.in, sc, t, ts);
-        r0 = rec_col(ts, 0);
-        r1 = rec_col(ts, 1);
-        r2 = rec_col(ts, 2);
-        if constexpr (NV > 0) Varyings<SHADER>::corners(a.in, sc, corner_slots(a.in, t), v);
-      }
-      const float x = pix_x(i, vp), y = pix_y(j, vp);
-      const float e[3] = {edge(r0, x, y), edge(r1, x, y), edge(r2, x, y)};
-      float wr = e[0] + e[1];
-      wr = wr + e[2];
-      const float b[3] = {e[0] / wr, e[1] / wr, e[2] / wr};
-      for (int k = 0; k < 3; ++k) {
-        g.db[k] = 0.0f;
-        for (int c = 0; c < 3; ++c) g.dvar[k][c] = 0.0f;
-      }
-      if (a.d_canvas || a.target) {
-        float dcol[3];
-        if (a.target) {
-          for (int c = 0; c < 3; ++c)
-            dcol[c] = a.l2_scale * (a.canvas[3 * pix + c] - a.target[3 * pix + c]);
-        } else {
-          for (int c = 0; c < 3; ++c) dcol[c] = a.d_canvas[3 * pix + c];
-        }
-        if constexpr (NV > 0)
-          ShadeBwd<SHADER>::run_v(a.in, sc, a.gr, v, b, dcol, g, s);
-        else
-          ShadeBwd<SHADER>::run(a.in, sc, a.gr, corner_slots(a.in, t), b, dcol, g, s);
-      }
-      // b = e / sum(e)
-      const float tdb = (g.db[0] * e[0] + g.db[1] * e[1]) + g.db[2] * e[2];
-      float de[3];
-      for (int k = 0; k < 3; ++k) de[k] = g.db[k] / wr - tdb / (wr * wr);
-      // zbuffer = (sum_k e_k z_k) * vp22 + vp23
-      if (a.d_zbuffer) {
-        const float dz = a.d_zbuffer[pix];
-        float zc = e[0] * r0.w;
-        zc = zc + e[1] * r1.w;
-        zc = zc + e[2] * r2.w;
-        const float zk[3] = {r0.w, r1.w, r2.w};
+        tri_setup(args().in, scene(), t, ts);
+        float* r = trec + lane * NS;
+#pragma unroll
         for (int k = 0; k < 3; ++k) {
-          de[k] += dz * vp[10] * zk[k];
-          vals[A_Z + k] = dz * vp[10] * e[k];
+          const float4 c = rec_col(ts, k);
+          r[4 * k + 0] = c.x;
+          r[4 * k + 1] = c.y;
+          r[4 * k + 2] = c.z;
+          r[4 * k + 3] = c.w;
         }
-        g.sg[S_VP22] += dz * zc;
-        g.sg[S_VP23] += dz;
       }
-      // e_k = x Minv[0][k] + y Minv[1][k] + Minv[2][k]
-      float dx = 0.0f, dy = 0.0f;
-      const float m0[3] = {r0.x, r1.x, r2.x}, m1[3] = {r0.y, r1.y, r2.y};
-      for (int k = 0; k < 3; ++k) {
-        vals[A_MINV + 0 * 3 + k] = x * de[k];
-        vals[A_MINV + 1 * 3 + k] = y * de[k];
-        vals[A_MINV + 2 * 3 + k] = de[k];
-        dx += m0[k] * de[k];
-        dy += m1[k] * de[k];
+    }
+    // the corner stage: one lane per corner of each listed triangle
+    if constexpr (NV > 0) {
+      for (int idx = lane; idx < 3 * CAP; idx += 64) {
+        const int e = idx / 3, k = idx - 3 * e;
+        const int32_t t = tab[e];
+        if (t >= 0)
+          V::corner(args().in, scene(), face_slot(args().in, t, k), face_slot(args().in, t, 0), k,
+                    trec + e * NS + 12);
       }
-      // x = (i - vp03) / vp00, y = (j - vp13) / vp11
-      g.sg[S_VP03] += -dx * ivp0;
-      g.sg[S_VP00] += -dx * x * ivp0;
-      g.sg[S_VP13] += -dy * ivp5;
-      g.sg[S_VP11] += -dy * y * ivp5;
-      for (int k = 0; k < 3; ++k)
-        for (int c = 0; c < 3; ++c) vals[A_VAR + 3 * k + c] = g.dvar[k][c];
-      if constexpr (DARBOUX) {
-        for (int k = 0; k < 9; ++k) vals[A_TRI + k] = g.dtri[k];
-        for (int k = 0; k < 6; ++k) vals[A_TUV + k] = g.dtuv[k];
+    }
+    __syncthreads();
+
+    uint32_t run_slot = 255u;  // the lane's open run and its sums
+    float run[NR];
+#pragma unroll
+    for (int k = 0; k < NR; ++k) run[k] = 0.0f;
+    auto flush_tri = [&]() {
+      if (run_slot != 255u) {
+        float* row = acc[run_slot];
+#pragma unroll
+        for (int k = 0; k < NR; ++k)
+          if (NV > 0 || k < R_VAR || k >= R_Z) atomicAdd(row + k, run[k]);
       }
-      for (int k = 0; k < ACC; ++k) run_v[k] += vals[k];
-    }
-    // texel and specular-map runs
-    if (g.tex_at != run_tex) {
-      stage_add<kTexCap, 3>(tex_tab, tex_val, a.gr.d_textures, run_tex, run_tex_n, run_tex_g,
-                            pend_tex);
-      run_tex = g.tex_at;
-      run_tex_n = g.tex_n;
-      run_tex_g[0] = run_tex_g[1] = run_tex_g[2] = 0.0f;
-    }
-    for (int c = 0; c < 3; ++c) run_tex_g[c] += g.tex_g[c];
-    if (g.spec_at != run_spec) {
-      stage_add<kSpecCap, 1>(spec_tab, spec_val, a.gr.d_specular_maps, run_spec, 1, &run_spec_g,
-                             pend_spec);
-      run_spec = g.spec_at;
-      run_spec_g = 0.0f;
-    }
-    run_spec_g += g.spec_g;
-    if constexpr (DARBOUX) {
-      if (g.nmap_at != run_nmap) {
-        stage_add<kNmapCap, 3>(nmap_tab, nmap_val, a.gr.d_normal_maps, run_nmap, 3, run_nmap_g,
-                               pend_nmap);
-        run_nmap = g.nmap_at;
-        run_nmap_g[0] = run_nmap_g[1] = run_nmap_g[2] = 0.0f;
-      }
-      for (int c = 0; c < 3; ++c) run_nmap_g[c] += g.nmap_g[c];
-    }
-  }
-  flush_tri();
-  stage_add<kTexCap, 3>(tex_tab, tex_val, a.gr.d_textures, run_tex, run_tex_n, run_tex_g,
-                        pend_tex);
-  stage_add<kSpecCap, 1>(spec_tab, spec_val, a.gr.d_specular_maps, run_spec, 1, &run_spec_g,
-                         pend_spec);
-  if constexpr (DARBOUX)
-    stage_add<kNmapCap, 3>(nmap_tab, nmap_val, a.gr.d_normal_maps, run_nmap, 3, run_nmap_g,
-                           pend_nmap);
-  if (a.gr.d_textures) pend_tex.flush(a.gr.d_textures);
-  if (a.gr.d_specular_maps) pend_spec.flush(a.gr.d_specular_maps);
-  if constexpr (DARBOUX)
-    if (a.gr.d_normal_maps) pend_nmap.flush(a.gr.d_normal_maps);
-  __syncthreads();
-  // one texel's channels: tex_c is the scene's (one scene per tile)
-  flush_adds<kTexCap, 3>(tex_tab, tex_val, a.gr.d_textures, sc.tex_c > 1 ? 3 : 1);
-  flush_adds<kSpecCap, 1>(spec_tab, spec_val, a.gr.d_specular_maps, 1);
-  if constexpr (DARBOUX) flush_adds<kNmapCap, 3>(nmap_tab, nmap_val, a.gr.d_normal_maps, 3);
-  if (lane < kBwdCap && tab[lane] >= 0) a.touched[tab[lane]] = s + 1;
-  // lanes take consecutive accumulators of a triangle's row: the addresses of
-  // one atomic instruction fall in few cache lines
-  for (int idx = lane; idx < kBwdCap * ACC; idx += 64) {
-    const int e = idx / ACC, k = idx - e * ACC;
-    const int32_t t = tab[e];
-    if (t < 0) continue;
-    const float v = acc[e][k];
-    if (v != 0.0f) atomicAdd(a.tacc + (int64_t)t * ACC + k, v);
-  }
-  // per-scene parameters: one reduction per tile.  The pixels summed the
-  // cotangents of normalise(light_direction) and normalise(light_dir_eye);
-  // normalise's backward is linear in them, so it is applied to the sums.
-  if (a.gr.d_scene) {
-    float tot[S_COUNT];
-    for (int q = 0; q < S_COUNT; ++q) tot[q] = wave_sum(g.sg[q]);
-    auto through_normalise = [&](const float* v, int at) {
-      if (tot[at] == 0.0f && tot[at + 1] == 0.0f && tot[at + 2] == 0.0f) return;
-      float d[3];
-      normalise_bwd(v, tot + at, d);
-      for (int q = 0; q < 3; ++q) tot[at + q] = d[q];
+#pragma unroll
+      for (int k = 0; k < NR; ++k) run[k] = 0.0f;
     };
-    through_normalise(sc.light_direction, S_LIGHT_DIR);
-    through_normalise(sc.light_dir_eye, S_LIGHT_DIR_EYE);
-    for (int q = 0; q < S_COUNT; ++q)
-      if (lane == 0 && tot[q] != 0.0f)
-        atomicAdd(a.gr.d_scene + (int64_t)s * JR_DSCENE_FLOATS + kSceneSlot[q], tot[q]);
+#pragma unroll 1
+    for (int q = 0; q < 4; ++q) {
+      const uint32_t slot = (slots >> (8 * q)) & 255u;
+      if (slot != run_slot) {
+        flush_tri();
+        run_slot = slot;
+      }
+      PixGrad<SHADER> g;
+      read_again();
+      if (slot != 255u) {
+        // the canvas cotangent, or the canvas and target that it is computed from:
+        // first, and used last
+        const int64_t pix = pix0 + (q >> 1) * args().H + (q & 1);
+        const float* from = args().target ? args().canvas : args().d_canvas;
+        float dcol[3] = {0.0f, 0.0f, 0.0f}, tgt[3] = {0.0f, 0.0f, 0.0f};
+        if (from) load3(from + 3 * pix, 0, dcol);
+        if (args().target) load3(args().target + 3 * pix, 0, tgt);
+        const float* r = trec + slot * NS;
+        const float* vary = r + 12;
+        const float x = q < 2 ? x0 : x1, y = q & 1 ? y1 : y0;
+        float4 col[3];
+        float e[3], b[3], db[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          col[k] = make_float4(r[4 * k], r[4 * k + 1], r[4 * k + 2], r[4 * k + 3]);
+          e[k] = edge(col[k], x, y);
+        }
+        float wr = e[0] + e[1];
+        wr = wr + e[2];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) b[k] = e[k] / wr;
+        if constexpr (NV > 0) {
+          if (from) {
+            if (args().target) {
+#pragma unroll
+              for (int c = 0; c < 3; ++c) dcol[c] = args().l2_scale * (dcol[c] - tgt[c]);
+            }
+            float n[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) n[c] = interp(b, vary[c], vary[3 + c], vary[6 + c]);
+            ShadeBwd<SHADER>::run(args().in, scene(), args().gr, vary, n, b, light, dcol, g,
+                                  sg, s);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+              db[k] = dot3(g.dn, vary + 3 * k);
+#pragma unroll
+              for (int c = 0; c < 3; ++c) run[R_VAR + 3 * k + c] += b[k] * g.dn[c];
+            }
+          }
+        }
+        // b = e / sum(e)
+        const float tdb = (db[0] * e[0] + db[1] * e[1]) + db[2] * e[2];
+        const float all = tdb / (wr * wr);
+        float de[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) de[k] = db[k] / wr - all;
+        // zbuffer = (sum_k e_k z_k) * vp22 + vp23
+        if constexpr (DZ) {
+          const float dz = args().d_zbuffer[pix], vp22 = scene().viewport[10];
+#pragma unroll
+          for (int k = 0; k < 3; ++k) {
+            de[k] += dz * vp22 * col[k].w;
+            run[R_Z + k] += dz * vp22 * e[k];
+          }
+          float zc = e[0] * col[0].w;
+          zc = zc + e[1] * col[1].w;
+          zc = zc + e[2] * col[2].w;
+          sg[NSH] += dz * zc;
+          sg[NSH + 1] += dz;
+        }
+        // e_k = x Minv[0][k] + y Minv[1][k] + Minv[2][k]
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          run[A_MINV + k] += x * de[k];
+          run[A_MINV + 3 + k] += y * de[k];
+          run[A_MINV + 6 + k] += de[k];
+        }
+        if constexpr (DARBOUX) {
+#pragma unroll
+          for (int k = 0; k < 15; ++k) run[R_TRI + k] += g.more[k];
+        }
+      }
+      if constexpr (NV > 9) {
+        const bool tex = g.u >= 0 && args().gr.d_textures;
+        const int64_t m = (int64_t)g.u * scene().tex_h + g.v;
+        if (scene().tex_c == 1) g.tex_g[0] = (g.tex_g[0] + g.tex_g[1]) + g.tex_g[2];
+        if (!huge) {
+          const int32_t key = tex ? (int32_t)(uint32_t)m : -1;
+          if (key != tex_key) {
+            if (tex_key != -1) tex_tab.add(tex_key, tex_sum, add_texel);
+            tex_key = key;
+#pragma unroll
+            for (int c = 0; c < NT; ++c) tex_sum[c] = 0.0f;
+          }
+#pragma unroll
+          for (int c = 0; c < 3; ++c) tex_sum[c] += tex ? g.tex_g[c] : 0.0f;
+          if constexpr (REFLECT) tex_sum[NT - 1] += one_map ? g.spec_g : 0.0f;
+        } else if (tex) {
+          for (int c = 0; c < 3; ++c) texel_at(m, c, g.tex_g[c]);
+        }
+        if constexpr (REFLECT || DARBOUX) {
+          if (g.us >= 0 && (huge || !one_map)) {
+            const int64_t k = (int64_t)g.us * (DARBOUX ? scene().nmap_h : scene().spec_h) + g.vs;
+            const float* mg = DARBOUX ? g.nmap_g : &g.spec_g;
+            if (!huge) {
+              map_tab.add((int32_t)(uint32_t)k, mg, add_entry);
+            } else {
+              for (int c = 0; c < N2; ++c) entry_at(k, c, mg[c]);
+            }
+          }
+        }
+      }
+    }
+    // The lanes' last runs: most end here, together.  An LDS atomic of n lanes on
+    // one triangle takes the LDS n turns for each of the sums, so a triangle that
+    // at least kShared lanes end on is summed across the wavefront first, and its
+    // sums are added by a lane each.  The search is bounded: a wavefront of small
+    // triangles has none to find.
+    {
+      uint64_t left = __ballot(run_slot != 255u);
+      for (int n = 0; n < kSearched && __popcll(left) >= kShared; ++n) {
+        const uint32_t one = __builtin_amdgcn_readlane(run_slot, __builtin_ctzll(left));
+        const uint64_t same = __ballot(run_slot == one);
+        left &= ~same;
+        if (__popcll(same) < kShared) continue;
+        const bool in = run_slot == one;
+        constexpr int N1 = NR < 32 ? NR : 18;
+        float v[N1];
+#pragma unroll
+        for (int k = 0; k < N1; ++k) v[k] = in ? run[k] : 0.0f;
+        const float tot = wave_totals(v);
+        if ((lane & 1) == 0 && (lane >> 1) < N1) atomicAdd(&acc[one][lane >> 1], tot);
+        if constexpr (NR > N1) {
+          float w[NR - N1];
+#pragma unroll
+          for (int k = 0; k < NR - N1; ++k) w[k] = in ? run[N1 + k] : 0.0f;
+          const float more = wave_totals(w);
+          if ((lane & 1) == 0 && (lane >> 1) < NR - N1)
+            atomicAdd(&acc[one][N1 + (lane >> 1)], more);
+        }
+        if (in) run_slot = 255u;
+      }
+    }
+    flush_tri();
+    read_again();
+    __syncthreads();
+    // the round's sums to memory: lanes take consecutive accumulators of a
+    // triangle's row, so that the addresses of one atomic instruction fall in
+    // few cache lines
+    if (lane < CAP && tab[lane] >= 0) args().touched[tab[lane]] = s + 1;
+    for (int idx = lane; idx < CAP * NR; idx += 64) {
+      const int e = idx / NR, r = idx - e * NR;
+      const int32_t t = tab[e];
+      if (t < 0) continue;
+      const float v = acc[e][r];
+      const int k = r < R_VAR ? r : r < R_Z ? r - R_VAR + A_VAR
+                                : r < R_TRI ? r - R_Z + A_Z : r - R_TRI + A_TRI;
+      if (v != 0.0f) atomicAdd(args().tacc + (int64_t)t * ACC + k, v);
+    }
+    __syncthreads();  // the next round writes over what was read here
+  }
+  if constexpr (NV > 9) {
+    // the lanes' last runs, as the triangles' above
+    uint64_t left = __ballot(tex_key != -1);
+    for (int n = 0; n < kTexSearched && __popcll(left) >= kTexShared; ++n) {
+      const int32_t one = __builtin_amdgcn_readlane(tex_key, __builtin_ctzll(left));
+      const uint64_t same = __ballot(tex_key == one);
+      left &= ~same;
+      if (__popcll(same) < kTexShared) continue;
+      const bool in = tex_key == one;
+      float v[NT];
+#pragma unroll
+      for (int c = 0; c < NT; ++c) v[c] = in ? tex_sum[c] : 0.0f;
+      const float tot = wave_totals(v);
+#pragma unroll
+      for (int c = 0; c < NT; ++c)
+        v[c] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(tot), 2 * c));
+      if (lane == 0) tex_tab.add(one, v, add_texel);
+      if (in) tex_key = -1;
+    }
+    if (tex_key != -1) tex_tab.add(tex_key, tex_sum, add_texel);
+    __syncthreads();
+    tex_tab.flush(add_texel);
+    if constexpr (REFLECT || DARBOUX)
+      if (!one_map) map_tab.flush(add_entry);
+  }
+  // per-scene parameters: one reduction per wavefront, lane 2 j taking sum j.  The
+  // pixels summed the cotangent of normalise(S_DIR's direction); normalise's
+  // backward is linear in it, so it is applied to the sum.
+  if (!args().gr.d_scene) return;
+  float* row = args().gr.d_scene + (int64_t)s * JR_DSCENE_FLOATS;
+  if constexpr (NSG > 0) {
+    const float tot = wave_totals(sg);
+    auto sum_of = [&](int j) {
+      return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(tot), 2 * j));
+    };
+    const int j = lane >> 1, q = j - 3 * (j / 3), group = j - q;
+    const bool mine = (lane & 1) == 0;
+    float v = tot;
+    int at = -1;
+    if (j >= NSH) {
+      at = JR_DSCENE_VIEWPORT + 10 + j - NSH;
+    } else if (group == S_DIR) {
+      const float dy[3] = {sum_of(S_DIR), sum_of(S_DIR + 1), sum_of(S_DIR + 2)};
+      float d[3] = {0.0f, 0.0f, 0.0f};
+      if (dy[0] != 0.0f || dy[1] != 0.0f || dy[2] != 0.0f)
+        normalise_bwd(REFLECT ? scene().light_dir_eye : scene().light_direction, dy, d);
+      v = q == 0 ? d[0] : q == 1 ? d[1] : d[2];
+      at = (REFLECT ? JR_DSCENE_LIGHT_DIR_EYE : JR_DSCENE_LIGHT_DIRECTION) + q;
+    } else if (REFLECT && group == S_DIFFUSE) {
+      v = tot * scene().light_colour[q];
+      at = JR_DSCENE_DIFFUSE + q;
+    } else if (REFLECT && group == S_SPECULAR) {
+      v = tot * scene().light_colour[q];
+      at = JR_DSCENE_SPECULAR + q;
+    } else if (REFLECT && group == S_AMBIENT) {
+      at = JR_DSCENE_AMBIENT + q;
+    } else if (REFLECT && group == S_STRENGTH) {
+      at = JR_DSCENE_SHADOW_STRENGTH + q;
+    } else {
+      at = JR_DSCENE_LIGHT_COLOUR + q;
+    }
+    if (mine && j < NSG && v != 0.0f) atomicAdd(row + at, v);
+    if constexpr (REFLECT) {  // the light's colour, by the diffuse sums' lanes
+      const float spec = __shfl(tot, (lane + 2 * (S_SPECULAR - S_DIFFUSE)) & 63);
+      v = fmaf(scene().diffuse[q], tot, scene().specular[q] * spec);
+      if (mine && j < NSH && group == S_DIFFUSE && v != 0.0f)
+        atomicAdd(row + JR_DSCENE_LIGHT_COLOUR + q, v);
+    }
   }
 }
 
 // vertex-stage backward of one slot for its varying cotangent dv: the
 // gradient dn of the slot's normal row *nrow_out (and for gouraud dc of its
-// colour row *crow_out; rows stay -1 when there is nothing to add)
+// colour row *crow_out; rows stay -1 when there is nothing to add).  dE: the
+// sums of the light's direction and colour for the shaders lit here, else of the
+// 3x3 rotation of world_to_eye_norm.
 template <int SHADER>
 JR_DEV void vertex_bwd(const BwdArgs& a, const jr_scene& sc, int32_t slot, const float dv[3],
-                       float* dW, float* dE, float* dLd, float* dLc, int64_t* nrow_out,
-                       float dn[3], int64_t* crow_out, float dc[3]) {
+                       float* dE, int64_t* nrow_out, float dn[3], int64_t* crow_out,
+                       float dc[3]) {
   if (SHADER == JR_SHADER_DEPTH) return;
   if (dv[0] == 0.0f && dv[1] == 0.0f && dv[2] == 0.0f) return;
   const jr_inputs& in = a.in;
@@ -1017,12 +1068,12 @@ JR_DEV void vertex_bwd(const BwdArgs& a, const jr_scene& sc, int32_t slot, const
       *crow_out = crow;
       for (int q = 0; q < 3; ++q) {
         dc[q] = dv[q] * sc.light_colour[q] * it;
-        dLc[q] += dv[q] * col[q] * it;
+        dE[3 + q] += dv[q] * col[q] * it;
         dI += dv[q] * col[q] * sc.light_colour[q];
       }
     } else {
       for (int q = 0; q < 3; ++q) {
-        dLc[q] += dv[q] * it;
+        dE[3 + q] += dv[q] * it;
         dI += dv[q] * sc.light_colour[q];
       }
     }
@@ -1032,7 +1083,7 @@ JR_DEV void vertex_bwd(const BwdArgs& a, const jr_scene& sc, int32_t slot, const
       dln[q] = dI * nn[q];
     }
     normalise_bwd(sc.light_direction, dln, dL);
-    for (int q = 0; q < 3; ++q) dLd[q] += dL[q];
+    for (int q = 0; q < 3; ++q) dE[q] += dL[q];
   } else {
     // ne = normalise((E @ [normalise(nn), 0])[:3])  (Camera.apply_vec)
     float u2[3];
@@ -1046,7 +1097,7 @@ JR_DEV void vertex_bwd(const BwdArgs& a, const jr_scene& sc, int32_t slot, const
       float s = 0.0f;
       for (int ii = 0; ii < 3; ++ii) {
         s += sc.world_to_eye_norm[4 * ii + jj] * dt3[ii];
-        dE[4 * ii + jj] += dt3[ii] * u2[jj];
+        dE[3 * ii + jj] += dt3[ii] * u2[jj];
       }
       du2[jj] = s;
     }
@@ -1092,9 +1143,17 @@ JR_DEV void wave_row_adds(WaveRows& W, float* __restrict__ d, int64_t row, const
 // wavefront of one scene reduces its camera and light gradients once.
 template <int SHADER>
 JR_DEV void bwd_tri(const BwdArgs& a, int32_t t, int32_t s, bool touched, WaveRows& W) {
-  float dW[16], dE[16], dLd[3], dLc[3];
-  for (int q = 0; q < 16; ++q) dW[q] = dE[q] = 0.0f;
-  for (int q = 0; q < 3; ++q) dLd[q] = dLc[q] = 0.0f;
+  // gradients of the scene's parameters: world_to_clip, the rotation of
+  // world_to_eye_norm (or the light of a vertex-lit shader) and the viewport's
+  // entries 0, 3, 5, 7
+  constexpr bool LIT = SHADER == JR_SHADER_GOURAUD || SHADER == JR_SHADER_GOURAUD_TEXTURE;
+  constexpr int NE = SHADER == JR_SHADER_DEPTH ? 0 : LIT ? 6 : 9;
+  float dS[16 + 4 + NE];
+#pragma unroll
+  for (int q = 0; q < 16 + 4 + NE; ++q) dS[q] = 0.0f;
+  float* dW = dS;
+  float* dV = dS + 16;
+  float* dE = dS + 20;
   if (__ballot(touched) == 0) return;  // nothing to add for this wavefront
   if (!touched) s = -1;
   constexpr int ACC = AccOf<SHADER>::N;
@@ -1127,6 +1186,19 @@ JR_DEV void bwd_tri(const BwdArgs& a, int32_t t, int32_t s, bool touched, WaveRo
           for (int k = 0; k < 3; ++k) s2 += XtG[3 * p + k] * X[3 * q + k];
           dM[3 * p + q] = -s2;
         }
+      // x = (i - vp03) / vp00, y = (j - vp13) / vp11: with dx = sum_k X[0][k] de_k at
+      // a pixel, sum x dx = sum_k X[0][k] G[0][k] and sum dx = sum_k X[0][k] G[2][k]
+      for (int k = 0; k < 3; ++k) {
+        dV[0] -= X[k] * v[A_MINV + k];
+        dV[1] -= X[k] * v[A_MINV + 6 + k];
+        dV[2] -= X[3 + k] * v[A_MINV + 3 + k];
+        dV[3] -= X[3 + k] * v[A_MINV + 6 + k];
+      }
+      const float* vp = a.scenes[s].viewport;
+      dV[0] /= vp[0];
+      dV[1] /= vp[0];
+      dV[2] /= vp[5];
+      dV[3] /= vp[5];
     }
   }
   // corner by corner, the lanes' position / normal / colour rows added
@@ -1151,7 +1223,7 @@ JR_DEV void bwd_tri(const BwdArgs& a, int32_t t, int32_t s, bool touched, WaveRo
         if (jj < 3) dp[jj] = s2;
       }
       const float dv[3] = {v[A_VAR + 3 * k], v[A_VAR + 3 * k + 1], v[A_VAR + 3 * k + 2]};
-      vertex_bwd<SHADER>(a, sc, slot, dv, dW, dE, dLd, dLc, &nrow, dn, &crow, dc);
+      vertex_bwd<SHADER>(a, sc, slot, dv, dE, &nrow, dn, &crow, dc);
     }
     if (a.gr.d_positions) wave_row_adds(W, a.gr.d_positions, prow, dp);
     if constexpr (SHADER != JR_SHADER_DEPTH)
@@ -1212,39 +1284,29 @@ JR_DEV void bwd_tri(const BwdArgs& a, int32_t t, int32_t s, bool touched, WaveRo
     }
   }
   if (!a.gr.d_scene) return;
+  // where dS[j] goes in a d_scene row
+  auto slot_of = [&](int j) {
+    if (j < 16) return JR_DSCENE_WORLD_TO_CLIP + j;
+    if (j < 20)  // 0, 3, 5, 7
+      return JR_DSCENE_VIEWPORT + (j == 16 ? 0 : 2 * (j - 16) + 1);
+    const int k = j - 20;
+    if (LIT)
+      return k < 3 ? JR_DSCENE_LIGHT_DIRECTION + k : JR_DSCENE_LIGHT_COLOUR + k - 3;
+    return JR_DSCENE_WORLD_TO_EYE_NORM + k + k / 3;  // 3x3 of a 4x4
+  };
   // reduce over the wave when it holds one scene, else per lane
   const int32_t s0 = __shfl(s, 0);
   const bool uniform = __ballot(s == s0 || s < 0) == __ballot(true) && s0 >= 0;
-  float* base = a.gr.d_scene;
   if (uniform) {
     const int lane = threadIdx.x & 63;
-    float* row = base + (int64_t)s0 * JR_DSCENE_FLOATS;
-    for (int q = 0; q < 16; ++q) {
-      const float w = wave_sum(dW[q]);
-      const float e = wave_sum(dE[q]);
-      if (lane == 0) {
-        if (w != 0.0f) atomicAdd(row + JR_DSCENE_WORLD_TO_CLIP + q, w);
-        if (e != 0.0f) atomicAdd(row + JR_DSCENE_WORLD_TO_EYE_NORM + q, e);
-      }
-    }
-    for (int q = 0; q < 3; ++q) {
-      const float l = wave_sum(dLd[q]);
-      const float c = wave_sum(dLc[q]);
-      if (lane == 0) {
-        if (l != 0.0f) atomicAdd(row + JR_DSCENE_LIGHT_DIRECTION + q, l);
-        if (c != 0.0f) atomicAdd(row + JR_DSCENE_LIGHT_COLOUR + q, c);
-      }
-    }
+    const float tot = wave_totals(dS);
+    if ((lane & 1) == 0 && (lane >> 1) < 20 + NE && tot != 0.0f)
+      atomicAdd(a.gr.d_scene + (int64_t)s0 * JR_DSCENE_FLOATS + slot_of(lane >> 1), tot);
   } else if (s >= 0) {
-    float* row = base + (int64_t)s * JR_DSCENE_FLOATS;
-    for (int q = 0; q < 16; ++q) {
-      if (dW[q] != 0.0f) atomicAdd(row + JR_DSCENE_WORLD_TO_CLIP + q, dW[q]);
-      if (dE[q] != 0.0f) atomicAdd(row + JR_DSCENE_WORLD_TO_EYE_NORM + q, dE[q]);
-    }
-    for (int q = 0; q < 3; ++q) {
-      if (dLd[q] != 0.0f) atomicAdd(row + JR_DSCENE_LIGHT_DIRECTION + q, dLd[q]);
-      if (dLc[q] != 0.0f) atomicAdd(row + JR_DSCENE_LIGHT_COLOUR + q, dLc[q]);
-    }
+    float* row = a.gr.d_scene + (int64_t)s * JR_DSCENE_FLOATS;
+#pragma unroll
+    for (int j = 0; j < 20 + NE; ++j)
+      if (dS[j] != 0.0f) atomicAdd(row + slot_of(j), dS[j]);
   }
 }
 
@@ -1309,7 +1371,10 @@ int32_t bfail(int32_t code, const char* msg) {
 template <int SHADER>
 void launch_bwd(const BwdArgs& a, hipStream_t st) {
   const int64_t n_waves = (int64_t)a.T * a.n_scenes;
-  hipLaunchKernelGGL(k_bwd_pixels<SHADER>, dim3((unsigned)n_waves), dim3(64), 0, st, a);
+  if (a.d_zbuffer)
+    hipLaunchKernelGGL((k_bwd_pixels<SHADER, true>), dim3((unsigned)n_waves), dim3(64), 0, st, a);
+  else
+    hipLaunchKernelGGL((k_bwd_pixels<SHADER, false>), dim3((unsigned)n_waves), dim3(64), 0, st, a);
   hipLaunchKernelGGL(k_bwd_tris<SHADER>, dim3((a.in.n_tris + 255) / 256), dim3(256), 0, st, a);
 }
 

@@ -1445,8 +1445,8 @@ JR_DEV void finish_tile_shared(const RasterArgs& a, const jr_scene& sc, int32_t 
   const int32_t nd = *n_dense;
   for (int32_t idx = tid; idx < 3 * nd; idx += NT) {
     const int32_t d = idx / 3, k = idx - 3 * d;
-    const int32_t e = dense[d];
-    V::corner(a.in, sc, corner_slots(a.in, tab[e]), k, vary + e * NS);
+    const int32_t e = dense[d], t = tab[e];
+    V::corner(a.in, sc, face_slot(a.in, t, k), face_slot(a.in, t, 0), k, vary + e * NS);
   }
   tile_sync<WAVE>();
   float l[3];

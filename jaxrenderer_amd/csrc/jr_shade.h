@@ -115,8 +115,10 @@ JR_DEV float shadow_get(const float* __restrict__ map, int32_t sw, int32_t sh,
   int32_t iy = f2i_sat(roundf(y));
   if (ix < 0) ix += sw;
   if (iy < 0) iy += sh;
-  if (ix < 0 || ix >= sw || iy < 0 || iy >= sh) return __builtin_inff();
-  return map[(int64_t)ix * sh + iy];
+  // the load is outside the test, so that it can be in flight with others
+  const bool in_map = ix >= 0 && ix < sw && iy >= 0 && iy < sh;
+  const float z = map[in_map ? (int64_t)ix * sh + iy : 0];
+  return in_map ? z : __builtin_inff();
 }
 
 // Depth of the shadow map at light-viewport position (x, y) of a scene, read
@@ -198,102 +200,6 @@ struct Shade<JR_SHADER_VISIBILITY> {
   }
 };
 
-
-
-
-// shaders/phong_darboux.py:116-293
-template <>
-struct Shade<JR_SHADER_PHONG_DARBOUX> {
-  static JR_DEV bool run(const jr_inputs& in, const jr_scene& sc,
-                         const Corner& c, const float b[3], bool front,
-                         float col[3], int) {
-    float ne[3][3], uvv[3][2];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      eye_normal(in, sc, c.slot[k], ne[k]);
-      load2(in.uvs, attr_row(in.uv_index, c.slot[k]), uvv[k]);
-    }
-    // triangle (NDC) and triangle_uv of the face of slot 0, not interpolated
-    const int32_t face = in.id_to_face[c.slot[0]];
-    float tri[3][3], tuv[3][2];
-#pragma unroll
-    for (int m = 0; m < 3; ++m) {
-      const int32_t q = in.face_slots[3 * (int64_t)face + m];
-      float h[4];
-      position_clip(in, sc.world_to_clip, q, h);
-      // to_cartesian: drop w without dividing when w == 0
-      const bool wz = (h[3] == 0.0f);
-      tri[m][0] = wz ? h[0] : h[0] / h[3];
-      tri[m][1] = wz ? h[1] : h[1] / h[3];
-      tri[m][2] = wz ? h[2] : h[2] / h[3];
-      load2(in.uvs, attr_row(in.uv_index, q), tuv[m]);
-    }
-    float n_i[3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) n_i[q] = interp(b, ne[0][q], ne[1][q], ne[2][q]);
-    const float uu = interp(b, uvv[0][0], uvv[1][0], uvv[2][0]);
-    const float vv = interp(b, uvv[0][1], uvv[1][1], uvv[2][1]);
-    const int32_t u = floor_mod(f2i_sat(floorf(uu)), sc.tex_w);
-    const int32_t v = floor_mod(f2i_sat(floorf(vv)), sc.tex_h);
-    float n[3];
-    normalise3(n_i, n);
-    float A[9], AI[9];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      A[q] = tri[1][q] - tri[0][q];
-      A[3 + q] = tri[2][q] - tri[0][q];
-      A[6 + q] = n[q];
-    }
-    inv3(A, AI);
-    const float du1 = tuv[1][0] - tuv[0][0], du2 = tuv[2][0] - tuv[0][0];
-    const float dv1 = tuv[1][1] - tuv[0][1], dv2 = tuv[2][1] - tuv[0][1];
-    float iv[3], jv[3];
-#pragma unroll
-    for (int r = 0; r < 3; ++r) {
-      float s = AI[3 * r + 0] * du1;
-      s = s + AI[3 * r + 1] * du2;
-      s = s + AI[3 * r + 2] * 0.0f;
-      iv[r] = s;
-      float t = AI[3 * r + 0] * dv1;
-      t = t + AI[3 * r + 1] * dv2;
-      t = t + AI[3 * r + 2] * 0.0f;
-      jv[r] = t;
-    }
-    float in_[3], jn[3];
-    normalise3(iv, in_);
-    normalise3(jv, jn);
-    // B = [normalise(i), normalise(j), n] as columns; B @ normal_map[u, v]
-    const int32_t un = index_clamp(u, sc.nmap_w);
-    const int32_t vn = index_clamp(v, sc.nmap_h);
-    float nm[3];
-    load3(in.normal_maps + sc.nmap_base, un * sc.nmap_h + vn, nm);
-    float bn[3];
-#pragma unroll
-    for (int r = 0; r < 3; ++r) {
-      float s = in_[r] * nm[0];
-      s = s + jn[r] * nm[1];
-      s = s + n[r] * nm[2];
-      bn[r] = s;
-    }
-    float n2[3], ln[3];
-    normalise3(bn, n2);
-    normalise3(sc.light_direction, ln);
-    const float d = dot3(n2, ln);
-    float tex[3];
-    tex_rgb(in.textures, sc.tex_base, sc.tex_h, sc.tex_c, u, v, tex);
-    float lc[3];
-    bool pos = true;
-#pragma unroll
-    for (int ch = 0; ch < 3; ++ch) {
-      lc[ch] = sc.light_colour[ch] * d;
-      pos = pos && (lc[ch] >= 0.0f);
-    }
-#pragma unroll
-    for (int ch = 0; ch < 3; ++ch) col[ch] = pos ? tex[ch] * lc[ch] : 0.0f;
-    return front;
-  }
-};
-
 // Shaders whose fragment stage splits into a per-triangle part (the vertex
 // stage outputs of the three corners, packed into N floats) and a per-pixel
 // part.  A tile computes the per-triangle part once for each distinct winning
@@ -308,15 +214,16 @@ struct Varyings {
 template <>
 struct Varyings<JR_SHADER_GOURAUD> {
   static constexpr int N = 9;
-  // corner k's entries of v (another lane may write the other corners')
-  static JR_DEV void corner(const jr_inputs& in, const jr_scene& sc, const Corner& c, int k,
-                            float* v) {
-    gouraud_vertex(in, sc, c.slot[k], v + 3 * k);
+  // corner k's entries of v (another lane may write the other corners'), the
+  // corner's slot and the triangle's first
+  static JR_DEV void corner(const jr_inputs& in, const jr_scene& sc, int32_t slot, int32_t,
+                            int k, float* v) {
+    gouraud_vertex(in, sc, slot, v + 3 * k);
   }
   static JR_DEV void corners(const jr_inputs& in, const jr_scene& sc, const Corner& c,
                              float v[N]) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k) corner(in, sc, c, k, v);
+    for (int k = 0; k < 3; ++k) corner(in, sc, c.slot[k], c.slot[0], k, v);
   }
   static JR_DEV void scene_terms(const jr_scene&, float l[3]) { l[0] = l[1] = l[2] = 0.0f; }
   static JR_DEV bool pixel(const jr_inputs&, const jr_scene&, const float v[N], const float*,
@@ -336,9 +243,9 @@ struct Varyings<JR_SHADER_GOURAUD> {
 template <>
 struct Varyings<JR_SHADER_GOURAUD_TEXTURE> {
   static constexpr int N = 15;
-  static JR_DEV void corner(const jr_inputs& in, const jr_scene& sc, const Corner& c, int k,
-                            float* v) {
-    const SlotRows r = slot_rows(in, c.slot[k]);
+  static JR_DEV void corner(const jr_inputs& in, const jr_scene& sc, int32_t slot, int32_t,
+                            int k, float* v) {
+    const SlotRows r = slot_rows(in, slot);
     float nn_l[3], n[3], nn[3];
     load3(in.normals, r.nrm, n);
     load2(in.uvs, r.uv, v + 9 + 2 * k);
@@ -352,7 +259,7 @@ struct Varyings<JR_SHADER_GOURAUD_TEXTURE> {
   static JR_DEV void corners(const jr_inputs& in, const jr_scene& sc, const Corner& c,
                              float v[N]) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k) corner(in, sc, c, k, v);
+    for (int k = 0; k < 3; ++k) corner(in, sc, c.slot[k], c.slot[0], k, v);
   }
   static JR_DEV void scene_terms(const jr_scene&, float l[3]) { l[0] = l[1] = l[2] = 0.0f; }
   static JR_DEV bool pixel(const jr_inputs& in, const jr_scene& sc, const float v[N],
@@ -382,9 +289,9 @@ struct Varyings<JR_SHADER_GOURAUD_TEXTURE> {
 template <>
 struct Varyings<JR_SHADER_PHONG> {
   static constexpr int N = 15;
-  static JR_DEV void corner(const jr_inputs& in, const jr_scene& sc, const Corner& c, int k,
-                            float* v) {
-    const SlotRows r = slot_rows(in, c.slot[k]);
+  static JR_DEV void corner(const jr_inputs& in, const jr_scene& sc, int32_t slot, int32_t,
+                            int k, float* v) {
+    const SlotRows r = slot_rows(in, slot);
     float n[3];
     load3(in.normals, r.nrm, n);
     load2(in.uvs, r.uv, v + 9 + 2 * k);
@@ -393,7 +300,7 @@ struct Varyings<JR_SHADER_PHONG> {
   static JR_DEV void corners(const jr_inputs& in, const jr_scene& sc, const Corner& c,
                              float v[N]) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k) corner(in, sc, c, k, v);
+    for (int k = 0; k < 3; ++k) corner(in, sc, c.slot[k], c.slot[0], k, v);
   }
   static JR_DEV void scene_terms(const jr_scene& sc, float l[3]) {
     normalise3(sc.light_direction, l);
@@ -427,6 +334,111 @@ struct Varyings<JR_SHADER_PHONG> {
   }
 };
 
+// shaders/phong_darboux.py:116-293: per corner the eye-space normal and the
+// uv; the NDC corners and uvs (not interpolated) of the face of slot 0.
+template <>
+struct Varyings<JR_SHADER_PHONG_DARBOUX> {
+  static constexpr int N = 30;
+  static constexpr int kTri = 15, kTuv = 24;
+  static JR_DEV void corner(const jr_inputs& in, const jr_scene& sc, int32_t slot,
+                            int32_t slot0, int k, float* v) {
+    eye_normal(in, sc, slot, v + 3 * k);
+    load2(in.uvs, attr_row(in.uv_index, slot), v + 9 + 2 * k);
+    const int32_t q = in.face_slots[3 * (int64_t)in.id_to_face[slot0] + k];
+    float h[4];
+    position_clip(in, sc.world_to_clip, q, h);
+    // to_cartesian: drop w without dividing when w == 0
+    const bool wz = (h[3] == 0.0f);
+    float* tri = v + kTri + 3 * k;
+    tri[0] = wz ? h[0] : h[0] / h[3];
+    tri[1] = wz ? h[1] : h[1] / h[3];
+    tri[2] = wz ? h[2] : h[2] / h[3];
+    load2(in.uvs, attr_row(in.uv_index, q), v + kTuv + 2 * k);
+  }
+  static JR_DEV void corners(const jr_inputs& in, const jr_scene& sc, const Corner& c,
+                             float v[N]) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) corner(in, sc, c.slot[k], c.slot[0], k, v);
+  }
+  static JR_DEV void scene_terms(const jr_scene& sc, float l[3]) {
+    normalise3(sc.light_direction, l);
+  }
+  // the tangent frame of a pixel with unit normal n: inv([t1 - t0; t2 - t0; n]) =: AI,
+  // (iv, jv) = AI @ (du, dv)
+  static JR_DEV void tangents(const float* v, const float n[3], float AI[9], float iv[3],
+                              float jv[3]) {
+    const float* tri = v + kTri;
+    const float* tuv = v + kTuv;
+    float A[9];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      A[q] = tri[3 + q] - tri[q];
+      A[3 + q] = tri[6 + q] - tri[q];
+      A[6 + q] = n[q];
+    }
+    inv3(A, AI);
+    const float du1 = tuv[2] - tuv[0], du2 = tuv[4] - tuv[0];
+    const float dv1 = tuv[3] - tuv[1], dv2 = tuv[5] - tuv[1];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      float s = AI[3 * r + 0] * du1;
+      s = s + AI[3 * r + 1] * du2;
+      s = s + AI[3 * r + 2] * 0.0f;
+      iv[r] = s;
+      float t = AI[3 * r + 0] * dv1;
+      t = t + AI[3 * r + 1] * dv2;
+      t = t + AI[3 * r + 2] * 0.0f;
+      jv[r] = t;
+    }
+  }
+  static JR_DEV bool pixel(const jr_inputs& in, const jr_scene& sc, const float v[N],
+                           const float ln[3], const float b[3], bool front, float col[3],
+                           int) {
+    const float* ne = v;
+    const float* uvv = v + 9;
+    float n_i[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) n_i[q] = interp(b, ne[q], ne[3 + q], ne[6 + q]);
+    const float uu = interp(b, uvv[0], uvv[2], uvv[4]);
+    const float vv = interp(b, uvv[1], uvv[3], uvv[5]);
+    const int32_t u = floor_mod(f2i_sat(floorf(uu)), sc.tex_w);
+    const int32_t t = floor_mod(f2i_sat(floorf(vv)), sc.tex_h);
+    float n[3], AI[9], iv[3], jv[3], in_[3], jn[3];
+    normalise3(n_i, n);
+    tangents(v, n, AI, iv, jv);
+    normalise3(iv, in_);
+    normalise3(jv, jn);
+    // B = [normalise(i), normalise(j), n] as columns; B @ normal_map[u, v]
+    const int32_t un = index_clamp(u, sc.nmap_w);
+    const int32_t vn = index_clamp(t, sc.nmap_h);
+    float nm[3];
+    load3(in.normal_maps + sc.nmap_base, un * sc.nmap_h + vn, nm);
+    float bn[3];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      float s = in_[r] * nm[0];
+      s = s + jn[r] * nm[1];
+      s = s + n[r] * nm[2];
+      bn[r] = s;
+    }
+    float n2[3];
+    normalise3(bn, n2);
+    const float d = dot3(n2, ln);
+    float tex[3];
+    tex_rgb(in.textures, sc.tex_base, sc.tex_h, sc.tex_c, u, t, tex);
+    float lc[3];
+    bool pos = true;
+#pragma unroll
+    for (int ch = 0; ch < 3; ++ch) {
+      lc[ch] = sc.light_colour[ch] * d;
+      pos = pos && (lc[ch] >= 0.0f);
+    }
+#pragma unroll
+    for (int ch = 0; ch < 3; ++ch) col[ch] = pos ? tex[ch] * lc[ch] : 0.0f;
+    return front;
+  }
+};
+
 // The shaders above, whole, for a pixel of the triangle with corners c.
 template <int SHADER>
 struct ShadeVaryings {
@@ -445,6 +457,8 @@ template <>
 struct Shade<JR_SHADER_GOURAUD_TEXTURE> : ShadeVaryings<JR_SHADER_GOURAUD_TEXTURE> {};
 template <>
 struct Shade<JR_SHADER_PHONG> : ShadeVaryings<JR_SHADER_PHONG> {};
+template <>
+struct Shade<JR_SHADER_PHONG_DARBOUX> : ShadeVaryings<JR_SHADER_PHONG_DARBOUX> {};
 
 // shaders/phong_reflection.py:100-235: per corner the eye-space normal and
 // uv; the texture index of corner 0.
@@ -454,15 +468,15 @@ struct Varyings<JR_SHADER_PHONG_REFLECTION> {
   static constexpr int kTi = 15;     // texture index of corner 0
   static constexpr int kShape = 16;  // its texture_shape row (2 ints)
   // corner k's entries of v; corner 0 also the triangle's texture index and shape
-  static JR_DEV void corner(const jr_inputs& in, const jr_scene& sc, const Corner& c, int k,
-                            float* v) {
-    const SlotRows r = slot_rows(in, c.slot[k]);
+  static JR_DEV void corner(const jr_inputs& in, const jr_scene& sc, int32_t slot, int32_t,
+                            int k, float* v) {
+    const SlotRows r = slot_rows(in, slot);
     float n[3];
     load3(in.normals, r.nrm, n);
     load2(in.uvs, r.uv, v + 9 + 2 * k);
     eye_normal_of(n, sc, v + 3 * k);
     if (k == 0) {
-      const int32_t ti = in.tex_index[attr_row(in.tex_index_index, c.slot[0])];
+      const int32_t ti = in.tex_index[attr_row(in.tex_index_index, slot)];
       v[kTi] = __int_as_float(ti);
       texture_shape(in, sc, ti, v + kShape, v + kShape + 1);
     }
@@ -470,7 +484,7 @@ struct Varyings<JR_SHADER_PHONG_REFLECTION> {
   static JR_DEV void corners(const jr_inputs& in, const jr_scene& sc, const Corner& c,
                              float v[N]) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k) corner(in, sc, c, k, v);
+    for (int k = 0; k < 3; ++k) corner(in, sc, c.slot[k], c.slot[0], k, v);
   }
   // per-scene terms of the pixel stage, computed once per tile
   static JR_DEV void scene_terms(const jr_scene& sc, float l[3]) {
@@ -506,9 +520,9 @@ struct Varyings<JR_SHADER_PHONG_REFLECTION_SHADOW> {
   static constexpr int N = 30;
   static constexpr int kTi = 27;
   static constexpr int kShape = 28;
-  static JR_DEV void corner(const jr_inputs& in, const jr_scene& sc, const Corner& c, int k,
-                            float* v) {
-    const SlotRows r = slot_rows(in, c.slot[k]);
+  static JR_DEV void corner(const jr_inputs& in, const jr_scene& sc, int32_t slot, int32_t,
+                            int k, float* v) {
+    const SlotRows r = slot_rows(in, slot);
     float n[3], p[3], h[4];
     load3(in.normals, r.nrm, n);
     load3(in.positions, r.pos, p);
@@ -521,7 +535,7 @@ struct Varyings<JR_SHADER_PHONG_REFLECTION_SHADOW> {
     v[15 + 4 * k + 2] = h[2] / h[3];
     v[15 + 4 * k + 3] = h[3] / h[3];
     if (k == 0) {
-      const int32_t ti = in.tex_index[attr_row(in.tex_index_index, c.slot[0])];
+      const int32_t ti = in.tex_index[attr_row(in.tex_index_index, slot)];
       v[kTi] = __int_as_float(ti);
       texture_shape(in, sc, ti, v + kShape, v + kShape + 1);
     }
@@ -529,7 +543,7 @@ struct Varyings<JR_SHADER_PHONG_REFLECTION_SHADOW> {
   static JR_DEV void corners(const jr_inputs& in, const jr_scene& sc, const Corner& c,
                              float v[N]) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k) corner(in, sc, c, k, v);
+    for (int k = 0; k < 3; ++k) corner(in, sc, c.slot[k], c.slot[0], k, v);
   }
   static JR_DEV void scene_terms(const jr_scene& sc, float l[3]) {
     normalise3(sc.light_dir_eye, l);

@@ -128,9 +128,46 @@ def test_backward_on_odd_frame_sizes(shader, size):
     _check_against_float64(shader, 0, *size)
 
 
-def _check_against_float64(shader, seed, W, H):
+# Ends of the backward's ranges: a wavefront's table of triangles (28 or 32) filled
+# more than once, by 64 triangles on one 16x16 tile, and one triangle that every
+# lane of every wavefront sums.  (A triangle h wide in the unit picture loses some
+# (2 / h)^2 roundings of 6e-8: 6e-6 at h = 0.25, two pixels of sixteen.)
+@pytest.mark.parametrize("shader", SHADERS, ids=lambda s: s.__name__)
+@pytest.mark.parametrize("n_tris, size", [(1, (48, 40)), (64, (16, 16))])
+def test_backward_many_triangles_and_one(shader, n_tris, size):
+    _check_against_float64(shader, 5, *size, n_tris)
+
+
+def _many(shader, seed, w, h, n_tris):
+    """The soup's inputs with small triangles, or one that covers the frame."""
+    cam, faces, extra, shadow_call = scenes.soup_inputs(shader, seed, w, h, n_tris=max(n_tris, 2))
+    pos = np.array(extra.position, np.float32)
+    rng = np.random.default_rng(seed)
+    for k, f in enumerate(np.asarray(faces)):
+        if n_tris > 1:  # 8 x 8 places, front-facing
+            at = np.array([-1.6 + 0.45 * (k % 8), -1.6 + 0.45 * (k // 8), 0.0])
+            pos[f] = at + np.array([[-0.24, -0.22, 0], [0.24, -0.21, 0], [-0.02, 0.26, 0]])
+            pos[f, 2] += rng.uniform(-0.1, 0.1, 3)
+        else:
+            pos[f] = np.array([[-9, -7, 0.3], [8, -7, -0.2], [0, 9, 0.1]]) - [0, 0, 3.0 * k]
+    extra = extra._replace(position=pos)
+    if hasattr(extra, "normal"):  # lit: gouraud draws no negative colour
+        extra = extra._replace(normal=(np.array([0.3, 0.5, 0.8]) + 0.2 * extra.normal).astype(
+            np.float32))
+        if hasattr(extra, "colour"):
+            extra = extra._replace(colour=np.abs(extra.colour) + np.float32(0.1))
+    if hasattr(extra, "specular_map"):
+        extra = extra._replace(specular_map=(1.0 + 0.75 * extra.specular_map).astype(np.float32))
+    if shadow_call is not None:
+        extra = extra._replace(shadow=extra.shadow._replace(
+            shadow_map=np.full((shadow_call.width, shadow_call.height), 0.5, np.float32)))
+    return cam, faces, extra
+
+
+def _check_against_float64(shader, seed, W, H, n_tris=None):
     dev = torch.device("cuda")
-    cam, faces, extra = _setup(shader, seed, W, H)
+    cam, faces, extra = (_setup(shader, seed, W, H) if n_tris is None
+                         else _many(shader, seed, W, H, n_tris))
     call = build_call(cam, shader, faces, extra, W, H, init_buffers=True)
     pid = _plan.run(call, prim_id=True)["prim_id"][0].cpu().numpy()
     assert (pid >= 0).sum() > 50

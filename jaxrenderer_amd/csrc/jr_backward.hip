@@ -564,7 +564,7 @@ struct BwdArgs {
   int32_t* touched;         // per triangle: its scene + 1 once a pixel adds to it, zero between calls
   uint32_t* header;         // workspace header (kHdr* words)
   int32_t W, H, n_scenes;
-  // the 2x2 pixel blocks of a scene (k_bwd_pixels), nq of them numbered:
+  // the 2x2 (or 1x2) pixel blocks of a scene (k_bwd_pixels), nq of them numbered:
   // FX x FY tiles of 8 x 8 blocks, rw and rh blocks left over right of and
   // below them; blocks [0, full_end) are the tiles', [full_end, bottom_end)
   // those below them; T wavefronts per scene
@@ -587,32 +587,34 @@ JR_DEV KernArgs<T> kernel_args() {
   return (KernArgs<T>)__builtin_amdgcn_kernarg_segment_ptr();
 }
 
-// A scene's pixels in 2x2 blocks, one wavefront per 64 consecutive blocks of
-// this enumeration: the full tiles of 8 x 8 blocks (16 x 16 pixels) first,
-// tile by tile, so that each is one wavefront with lane l owning the block
-// (16 tx + 2 (l / 8), 16 ty + 2 (l % 8)); then the blocks below them (rh per
-// row) and those right of them (rw per column), which share wavefronts
-// instead of leaving most lanes of a partial tile idle (an 84 x 84 frame
-// takes 28 wavefronts, not 36).  Where that saves few wavefronts every tile,
-// partial ones included, is a wavefront of its own.
+// A scene's pixels in blocks of 2x2 (PPL = 4) or 1x2 (PPL = 2), one wavefront per
+// 64 consecutive blocks of this enumeration: the full tiles of 8 x 8 blocks first,
+// tile by tile, so that each is one wavefront with lane l owning the block (8 tx +
+// l / 8, 8 ty + l % 8); then the blocks below them (rh per row) and those right of
+// them (rw per column), which share wavefronts instead of leaving most lanes of a
+// partial tile idle (an 84 x 84 frame takes 28 wavefronts, not 36).  Where that
+// saves few wavefronts every tile, partial ones included, is a wavefront of its own.
 //
-// A wavefront works in rounds of up to tri_cap() distinct triangles (mostly one):
-// their setup and corner stage, by one lane per triangle and per corner, go to
-// LDS; then each lane goes over its four pixels.  A lane sums consecutive pixels of
-// one triangle, and of one texel, in registers and adds a run to the LDS sums when
-// it ends, so neighbouring pixels, which mostly share both, cost one LDS atomic
-// instead of four; the LDS sums reach memory once per (wavefront, triangle) and
-// (wavefront, map entry).
+// A wavefront that shows no triangle leaves at once.  The others work in rounds of
+// up to tri_cap() distinct triangles (mostly one round): their corners' clip
+// positions and corner stage, one lane per corner, and their setup, one lane per
+// triangle, go to LDS; then each lane goes over its pixels.  A lane sums
+// consecutive pixels of one triangle, and of one texel, in registers and adds a run
+// to the LDS sums when it ends, so neighbouring pixels, which mostly share both,
+// cost one LDS atomic instead of four; the LDS sums reach memory once per
+// (wavefront, triangle) and (wavefront, map entry).
 //
-// What bounds it: the LDS and round trips to memory.  The LDS takes a turn for
-// each lane of an atomic on one address, and half of a 480x270 frame's wavefronts
-// see one or two large triangles: 512 of them spent 2,470 LDS cycles per wavefront
-// beside 700 cycles' worth of VALU issue.  With the lanes' last runs summed across
-// the wavefront (1,320 LDS cycles), a fourth wavefront per SIMD (162 registers ->
-// 128: scalars read again for each pixel instead of spilt into vector registers,
-// no own path for triangles beyond the table) and the scene's sums reduced
-// together, k_bwd_pixels went from 2,972 to 2,238 us on those 512 frames and the
-// step from 5,205 to 4,465 us; 23 views of 201x187 216 -> 202 us.
+// What bounds it: round trips to memory, then the LDS, which takes a turn for each
+// lane of an atomic on one address.  On 512 frames of 480x270, where half of the
+// wavefronts show nothing and half of the others one large triangle, and where it
+// took 2,972 us: with the lanes' last runs summed across the wavefront (2,470 ->
+// 1,320 LDS cycles per wavefront), a fourth wavefront per SIMD (162 registers ->
+// 128: scalars read again for each pixel instead of spilt into vector registers, no
+// own path for triangles beyond the table) and the scene's sums reduced together,
+// 2,238 us; with the empty wavefronts gone at once, one chain of loads for corners
+// and setup, and triangles numbered, so that only those there are are cleared and
+// added, 1,758 us.  1,024 frames of 84x84: 573, 590, 538 us.
+//
 // 16 workgroups' LDS on a CU, 4 wavefronts per SIMD as 128 registers allow, takes
 // at most 10 KiB each.
 constexpr int tri_cap(int shader) {
@@ -625,13 +627,15 @@ constexpr int tex_cap(int shader) { return reflects(shader) ? 128 : 224; }
 // Lanes on one triangle (texel) from which a sum across the wavefront (some 95
 // instructions for 18 sums, 40 for 4) replaces their LDS atomics, and how many
 // triangles (texels) are looked at.
-constexpr int kShared = 8, kSearched = 8;
+constexpr int kShared = 4, kSearched = 12;
 constexpr int kTexShared = 16, kTexSearched = 4;
 constexpr int kMapCap = 32;  // entries of a second map (normal map, specular map)
 
-template <int SHADER, bool DZ>
+template <int SHADER, bool DZ, int PPL>
 __global__ __launch_bounds__(64)
-__attribute__((amdgpu_waves_per_eu(SHADER == JR_SHADER_PHONG_DARBOUX ? 2 : 4, 8))) void k_bwd_pixels(BwdArgs) {
+__attribute__((amdgpu_waves_per_eu(SHADER == JR_SHADER_PHONG_DARBOUX ? 2 : 4, 8)))
+void k_bwd_pixels(BwdArgs) {
+  constexpr int BW = PPL / 2;  // a lane's block is BW x 2 pixels
   using V = Varyings<SHADER>;
   constexpr int NV = V::N;
   constexpr int NS = (12 + NV) | 1;  // record stride (odd: no LDS bank conflicts)
@@ -648,7 +652,7 @@ __attribute__((amdgpu_waves_per_eu(SHADER == JR_SHADER_PHONG_DARBOUX ? 2 : 4, 8)
   constexpr int N2 = DARBOUX ? 3 : 1;
   __shared__ float trec[CAP * NS];
   __shared__ float acc[CAP][AS];
-  __shared__ int32_t tab[CAP];
+  __shared__ int32_t tab[CAP], ids[CAP];
   __shared__ float light[3];
   __shared__ SumTable<(NV > 9 ? tex_cap(SHADER) : 1), NT> tex_tab;
   __shared__ SumTable<DARBOUX || REFLECT ? kMapCap : 1, N2> map_tab;
@@ -671,26 +675,36 @@ __attribute__((amdgpu_waves_per_eu(SHADER == JR_SHADER_PHONG_DARBOUX ? 2 : 4, 8)
   if (Q < args().full_end) {  // a full tile per wavefront, its blocks row by row
     const int32_t tile = Q >> 6;
     const int32_t tx = udiv31(tile, args().fy_m, args().fy_sh), ty = tile - tx * args().FY;
-    bi = 16 * tx + 2 * ((Q >> 3) & 7);
+    bi = BW * (8 * tx + ((Q >> 3) & 7));
     bj = 16 * ty + 2 * (Q & 7);
   } else if (Q < args().bottom_end) {  // below the full tiles, rh blocks per row
     const int32_t q = Q - args().full_end;
     const int32_t row = udiv31(q, args().rh_m, args().rh_sh);
-    bi = 2 * row;
+    bi = BW * row;
     bj = 16 * args().FY + 2 * (q - row * args().rh);
   } else {  // right of them over the whole height, rw blocks per column
     const int32_t q = Q - args().bottom_end;
     const int32_t col = udiv31(q, args().rw_m, args().rw_sh);
-    bi = 16 * args().FX + 2 * (q - col * args().rw);
+    bi = BW * (8 * args().FX + (q - col * args().rw));
     bj = 2 * col;
   }
   sp = args().scenes + s;
   const int64_t pix0 = (int64_t)s * args().W * args().H + (int64_t)bi * args().H + bj;
-  // the block's pixels, q = 2 (i - bi) + (j - bj), that are in the picture
+  // the block's pixels, q = 2 (i - bi) + (j - bj), that show a triangle
+  auto pixel = [&](int q) { return pix0 + (q >> 1) * args().H + (q & 1); };
   uint32_t todo = 0u;
-  if (Q < args().nq && bi < args().W && bj < args().H)
-    todo = 1u | (bj + 1 < args().H ? 2u : 0u) | (bi + 1 < args().W ? 4u : 0u) |
-           (bi + 1 < args().W && bj + 1 < args().H ? 8u : 0u);
+  {
+    int32_t t[PPL];
+#pragma unroll
+    for (int q = 0; q < PPL; ++q) {
+      const bool in = Q < args().nq && bi + (q >> 1) < args().W && bj + (q & 1) < args().H;
+      t[q] = in ? args().prim_id[pixel(q)] : -1;
+    }
+#pragma unroll
+    for (int q = 0; q < PPL; ++q)
+      todo |= t[q] >= 0 && t[q] < args().in.n_tris ? 1u << q : 0u;
+  }
+  if (__ballot(todo != 0u) == 0) return;
   const float* vp = scene().viewport;
   const float x0 = pix_x(bi, vp), x1 = pix_x(bi + 1, vp);
   const float y0 = pix_y(bj, vp), y1 = pix_y(bj + 1, vp);
@@ -739,56 +753,64 @@ __attribute__((amdgpu_waves_per_eu(SHADER == JR_SHADER_PHONG_DARBOUX ? 2 : 4, 8)
 
   while (__ballot(todo != 0u) != 0) {
     read_again();
-    // the round's distinct triangles
+    // the round's distinct triangles: an LDS set, whose entries are then numbered
     if (lane < CAP) tab[lane] = -1;
-    for (int k = lane; k < CAP * AS; k += 64) (&acc[0][0])[k] = 0.0f;
     __syncthreads();
-    int32_t t4[4];
+    int32_t t4[PPL];
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-      t4[q] = (todo >> q) & 1u ? args().prim_id[pix0 + (q >> 1) * args().H + (q & 1)] : -1;
-    uint32_t slots = 0u;  // per pixel its triangle's table entry, 255: not in this round
-    int32_t last = -1, last_e = 255;
+    for (int q = 0; q < PPL; ++q) t4[q] = (todo >> q) & 1u ? args().prim_id[pixel(q)] : -1;
+    int32_t entry[PPL];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int32_t t = t4[q] < args().in.n_tris ? t4[q] : -1;
-      if (t < 0) {
-        todo &= ~(1u << q);  // background
-        slots |= 255u << (8 * q);
-        continue;
-      }
-      if (t != last) {
-        last = t;
-        last_e = table_insert(tab, CAP, t) & 255;
-      }
-      slots |= (uint32_t)last_e << (8 * q);
-      if (last_e != 255) todo &= ~(1u << q);
+    for (int q = 0; q < PPL; ++q) {
+      entry[q] = -1;
+      if (t4[q] >= 0)
+        entry[q] = q > 0 && t4[q] == t4[q > 0 ? q - 1 : 0] ? entry[q > 0 ? q - 1 : 0]
+                                                          : table_insert(tab, CAP, t4[q]);
     }
     __syncthreads();
-    if (lane < CAP) {
-      const int32_t t = tab[lane];
-      if (t >= 0) {
-        TriSetup ts;
-        tri_setup(args().in, scene(), t, ts);
-        float* r = trec + lane * NS;
+    const int32_t found = lane < CAP ? tab[lane] : -1;
+    const uint64_t used = __ballot(found >= 0);
+    const int32_t nt = __popcll(used);
+    const int32_t rank = __builtin_amdgcn_mbcnt_hi(
+        (uint32_t)(used >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)used, 0u));
+    if (found >= 0) ids[rank] = found;
+    uint32_t slots = 0u;  // per pixel the number of its triangle, 255: not in this round
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          const float4 c = rec_col(ts, k);
-          r[4 * k + 0] = c.x;
-          r[4 * k + 1] = c.y;
-          r[4 * k + 2] = c.z;
-          r[4 * k + 3] = c.w;
-        }
-      }
+    for (int q = 0; q < PPL; ++q) {
+      const int32_t r = __shfl(rank, entry[q] & 63);
+      slots |= (entry[q] >= 0 ? (uint32_t)r : 255u) << (8 * q);
+      if (entry[q] >= 0) todo &= ~(1u << q);
     }
-    // the corner stage: one lane per corner of each listed triangle
-    if constexpr (NV > 0) {
-      for (int idx = lane; idx < 3 * CAP; idx += 64) {
-        const int e = idx / 3, k = idx - 3 * e;
-        const int32_t t = tab[e];
-        if (t >= 0)
-          V::corner(args().in, scene(), face_slot(args().in, t, k), face_slot(args().in, t, 0), k,
-                    trec + e * NS + 12);
+    for (int k = lane; k < nt * AS; k += 64) (&acc[0][0])[k] = 0.0f;
+    __syncthreads();
+    // per corner, one lane each: its clip position (where the triangle's record goes
+    // next) and its corner stage, whose loads are in flight together
+    for (int idx = lane; idx < 3 * nt; idx += 64) {
+      const int e = idx / 3, k = idx - 3 * e;
+      const int32_t t = ids[e], slot = face_slot(args().in, t, k);
+      float* row = trec + e * NS;
+      float h[4];
+      position_clip(args().in, scene().world_to_clip, slot, h);
+      if constexpr (NV > 0)
+        V::corner(args().in, scene(), slot, face_slot(args().in, t, 0), k, row + 12);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) row[4 * k + c] = h[c];
+    }
+    __syncthreads();
+    if (lane < nt) {
+      TriSetup ts;
+      float* r = trec + lane * NS;
+#pragma unroll
+      for (int k = 0; k < 12; ++k) ts.clip[k / 4][k % 4] = r[k];
+      ts.det = tri_det(ts.clip, ts.M);
+      tri_finish(ts);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const float4 c = rec_col(ts, k);
+        r[4 * k + 0] = c.x;
+        r[4 * k + 1] = c.y;
+        r[4 * k + 2] = c.z;
+        r[4 * k + 3] = c.w;
       }
     }
     __syncthreads();
@@ -808,8 +830,9 @@ __attribute__((amdgpu_waves_per_eu(SHADER == JR_SHADER_PHONG_DARBOUX ? 2 : 4, 8)
       for (int k = 0; k < NR; ++k) run[k] = 0.0f;
     };
 #pragma unroll 1
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < PPL; ++q) {
       const uint32_t slot = (slots >> (8 * q)) & 255u;
+      if (__ballot(slot != 255u) == 0) continue;
       if (slot != run_slot) {
         flush_tri();
         run_slot = slot;
@@ -819,7 +842,7 @@ __attribute__((amdgpu_waves_per_eu(SHADER == JR_SHADER_PHONG_DARBOUX ? 2 : 4, 8)
       if (slot != 255u) {
         // the canvas cotangent, or the canvas and target that it is computed from:
         // first, and used last
-        const int64_t pix = pix0 + (q >> 1) * args().H + (q & 1);
+        const int64_t pix = pixel(q);
         const float* from = args().target ? args().canvas : args().d_canvas;
         float dcol[3] = {0.0f, 0.0f, 0.0f}, tgt[3] = {0.0f, 0.0f, 0.0f};
         if (from) load3(from + 3 * pix, 0, dcol);
@@ -956,11 +979,10 @@ __attribute__((amdgpu_waves_per_eu(SHADER == JR_SHADER_PHONG_DARBOUX ? 2 : 4, 8)
     // the round's sums to memory: lanes take consecutive accumulators of a
     // triangle's row, so that the addresses of one atomic instruction fall in
     // few cache lines
-    if (lane < CAP && tab[lane] >= 0) args().touched[tab[lane]] = s + 1;
-    for (int idx = lane; idx < CAP * NR; idx += 64) {
+    if (lane < nt) args().touched[ids[lane]] = s + 1;
+    for (int idx = lane; idx < nt * NR; idx += 64) {
       const int e = idx / NR, r = idx - e * NR;
-      const int32_t t = tab[e];
-      if (t < 0) continue;
+      const int32_t t = ids[e];
       const float v = acc[e][r];
       const int k = r < R_VAR ? r : r < R_Z ? r - R_VAR + A_VAR
                                 : r < R_TRI ? r - R_Z + A_Z : r - R_TRI + A_TRI;
@@ -1369,12 +1391,15 @@ int32_t bfail(int32_t code, const char* msg) {
 }
 
 template <int SHADER>
-void launch_bwd(const BwdArgs& a, hipStream_t st) {
+void launch_bwd(const BwdArgs& a, int ppl, hipStream_t st) {
   const int64_t n_waves = (int64_t)a.T * a.n_scenes;
+  const dim3 grid((unsigned)n_waves);
   if (a.d_zbuffer)
-    hipLaunchKernelGGL((k_bwd_pixels<SHADER, true>), dim3((unsigned)n_waves), dim3(64), 0, st, a);
+    hipLaunchKernelGGL((k_bwd_pixels<SHADER, true, 4>), grid, dim3(64), 0, st, a);
+  else if (ppl == 4)
+    hipLaunchKernelGGL((k_bwd_pixels<SHADER, false, 4>), grid, dim3(64), 0, st, a);
   else
-    hipLaunchKernelGGL((k_bwd_pixels<SHADER, false>), dim3((unsigned)n_waves), dim3(64), 0, st, a);
+    hipLaunchKernelGGL((k_bwd_pixels<SHADER, false, 2>), grid, dim3(64), 0, st, a);
   hipLaunchKernelGGL(k_bwd_tris<SHADER>, dim3((a.in.n_tris + 255) / 256), dim3(256), 0, st, a);
 }
 
@@ -1466,7 +1491,17 @@ int32_t backward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* s
   a.W = fr->width;
   a.H = fr->height;
   a.n_scenes = fr->n_scenes;
-  const int64_t QW = (a.W + 1) / 2, QH = (a.H + 1) / 2, nq = QW * QH;
+  // Four pixels per lane (16 x 16 tiles) or two (8 x 16).  Two halve a wavefront's
+  // chain of lookups and its triangles, for half as many pixels to pay for them: the
+  // faster one where the wavefronts of four are few rounds of the 4,096 that the
+  // chip holds and a tile has triangles to set up (23 views of 201x187, 3,600 such
+  // wavefronts, 190 -> 167 us; 64 of 256x256, 16,000, 411 -> 381 us; 256 scenes of
+  // 128x128 790 -> 759 us), but not where the picture is larger (512 of 480x270,
+  // 261,000 wavefronts, 4,100 against 4,480 us; 1,024 of 84x84, 29,000, 1,399 against
+  // 1,428 us) or its triangles are (64 views of a 200-triangle ball 258 against 274).
+  const int64_t tiles4 = (int64_t)((a.W + 15) / 16) * ((a.H + 15) / 16) * a.n_scenes;
+  const int ppl = !d_zbuffer && tiles4 <= 24576 && in->n_tris >= 4 * tiles4 ? 2 : 4;
+  const int64_t QW = (a.W + ppl / 2 - 1) / (ppl / 2), QH = (a.H + 1) / 2, nq = QW * QH;
   const int64_t tiles_y = (QH + 7) / 8, tiles = (QW + 7) / 8 * tiles_y;
   // the leftover blocks are packed where that saves at least an eighth of the
   // wavefronts (84 x 84: 28 instead of 36, fwd+bwd 1.58 -> 1.52 ms on 1024
@@ -1507,13 +1542,13 @@ int32_t backward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* s
                      dim3(256), 0, st, a.header,
                      reinterpret_cast<uint32_t*>(ws + WL.touched), nwords);
   switch (sh) {
-    case JR_SHADER_DEPTH: launch_bwd<JR_SHADER_DEPTH>(a, st); break;
-    case JR_SHADER_GOURAUD: launch_bwd<JR_SHADER_GOURAUD>(a, st); break;
-    case JR_SHADER_GOURAUD_TEXTURE: launch_bwd<JR_SHADER_GOURAUD_TEXTURE>(a, st); break;
-    case JR_SHADER_PHONG: launch_bwd<JR_SHADER_PHONG>(a, st); break;
-    case JR_SHADER_PHONG_DARBOUX: launch_bwd<JR_SHADER_PHONG_DARBOUX>(a, st); break;
-    case JR_SHADER_PHONG_REFLECTION: launch_bwd<JR_SHADER_PHONG_REFLECTION>(a, st); break;
-    default: launch_bwd<JR_SHADER_PHONG_REFLECTION_SHADOW>(a, st); break;
+    case JR_SHADER_DEPTH: launch_bwd<JR_SHADER_DEPTH>(a, ppl, st); break;
+    case JR_SHADER_GOURAUD: launch_bwd<JR_SHADER_GOURAUD>(a, ppl, st); break;
+    case JR_SHADER_GOURAUD_TEXTURE: launch_bwd<JR_SHADER_GOURAUD_TEXTURE>(a, ppl, st); break;
+    case JR_SHADER_PHONG: launch_bwd<JR_SHADER_PHONG>(a, ppl, st); break;
+    case JR_SHADER_PHONG_DARBOUX: launch_bwd<JR_SHADER_PHONG_DARBOUX>(a, ppl, st); break;
+    case JR_SHADER_PHONG_REFLECTION: launch_bwd<JR_SHADER_PHONG_REFLECTION>(a, ppl, st); break;
+    default: launch_bwd<JR_SHADER_PHONG_REFLECTION_SHADOW>(a, ppl, st); break;
   }
   const hipError_t err = hipGetLastError();
   if (err != hipSuccess) return bfail(JR_E_HIP, hipGetErrorString(err));

@@ -14,7 +14,7 @@ import pytest
 import torch
 
 from jaxrenderer_amd import _hip, _plan
-from jaxrenderer_amd.autograd import render_differentiable
+from jaxrenderer_amd.autograd import RenderFunction, render_differentiable
 from jaxrenderer_amd.geometry import Camera
 from jaxrenderer_amd.pipeline import build_call
 from jaxrenderer_amd.shaders import (
@@ -136,6 +136,30 @@ def test_backward_on_odd_frame_sizes(shader, size):
 @pytest.mark.parametrize("n_tris, size", [(1, (48, 40)), (64, (16, 16))])
 def test_backward_many_triangles_and_one(shader, n_tris, size):
     _check_against_float64(shader, 5, *size, n_tris)
+
+
+# Without a depth gradient the pixels take another instance of the kernel, with two
+# or four pixels per lane (a tile of at least four triangles in a small call has
+# two): against the one above, which sums the same terms in another order.
+@pytest.mark.parametrize("shader", [s for s in SHADERS if s is not DepthShader],
+                         ids=lambda s: s.__name__)
+@pytest.mark.parametrize("n_tris, size", [(1, (48, 40)), (64, (16, 16)), (None, (37, 29)),
+                                          (None, (19, 70))])
+def test_backward_without_depth_gradient(shader, n_tris, size):
+    dev = torch.device("cuda")
+    cam, faces, extra = (_setup(shader, 6, *size) if n_tris is None
+                         else _many(shader, 6, *size, n_tris))
+    L, cam32, extra32 = _leaves(cam, extra, torch.float32, dev)
+    zb, cv = render_differentiable(cam32, shader, faces, extra32, *size)
+    wc = torch.as_tensor(np.random.default_rng(7).normal(size=(*size, 3))).to(dev).float()
+    ctx = cv.grad_fn.next_functions[0][0]
+    both = RenderFunction.backward(ctx, torch.zeros_like(zb)[None], wc[None])
+    alone = RenderFunction.backward(ctx, None, wc[None])
+    assert sum(a is not None for a in both) >= 4
+    for k, (a, b) in enumerate(zip(both, alone)):
+        assert (a is None) == (b is None)
+        if a is not None:
+            assert float((a - b).norm()) <= 1e-4 * float(a.norm()), k
 
 
 def _many(shader, seed, w, h, n_tris):

@@ -626,8 +626,11 @@ constexpr int tri_cap(int shader) {
 constexpr int tex_cap(int shader) { return reflects(shader) ? 128 : 224; }
 // Lanes on one triangle (texel) from which a sum across the wavefront (some 95
 // instructions for 18 sums, 40 for 4) replaces their LDS atomics, and how many
-// triangles (texels) are looked at.
-constexpr int kShared = 4, kSearched = 12;
+// triangles (texels) are looked at.  Four lanes pay for it (64 gouraud views 411
+// against 426 us), but with four pixels to a lane, where it makes no difference
+// (512 frames of 480x270), eight leave the order of small triangles' sums as it was.
+constexpr int shared_from(int ppl) { return ppl == 4 ? 8 : 4; }
+constexpr int kSearched = 12;
 constexpr int kTexShared = 16, kTexSearched = 4;
 constexpr int kMapCap = 32;  // entries of a second map (normal map, specular map)
 
@@ -636,6 +639,7 @@ __global__ __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(SHADER == JR_SHADER_PHONG_DARBOUX ? 2 : 4, 8)))
 void k_bwd_pixels(BwdArgs) {
   constexpr int BW = PPL / 2;  // a lane's block is BW x 2 pixels
+  constexpr int kShared = shared_from(PPL);
   using V = Varyings<SHADER>;
   constexpr int NV = V::N;
   constexpr int NS = (12 + NV) | 1;  // record stride (odd: no LDS bank conflicts)
@@ -785,6 +789,7 @@ void k_bwd_pixels(BwdArgs) {
     __syncthreads();
     // per corner, one lane each: its clip position (where the triangle's record goes
     // next) and its corner stage, whose loads are in flight together
+#pragma unroll 1
     for (int idx = lane; idx < 3 * nt; idx += 64) {
       const int e = idx / 3, k = idx - 3 * e;
       const int32_t t = ids[e], slot = face_slot(args().in, t, k);

@@ -76,11 +76,12 @@ class RenderFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, call: RasterCall, params, positions, normals, colours, textures,
                 specular_maps, uvs=None, normal_maps=None):
-        dev = params.device
+        dev = positions.device  # params may stay on the host, where they are read
+        ctx.set_materialize_grads(False)
         rows = params.detach().float().cpu().numpy()
         scenes = _raster.scenes_to_device(scenes_with_rows(call.scenes, rows), dev)
-        inputs = {k: _plan.to_device(v, dev, k) for k, v in call.inputs.items()
-                  if k not in _TENSOR_INPUTS}
+        inputs = _plan.upload({k: v for k, v in call.inputs.items() if k not in _TENSOR_INPUTS},
+                              dev)
         tensors = (positions, normals, colours, textures, specular_maps, uvs, normal_maps)
         for name, t in zip(_TENSOR_INPUTS, tensors):
             if t is not None:
@@ -131,6 +132,21 @@ class RenderFunction(torch.autograd.Function):
         return (None, grads["d_scene"]) + tuple(grads[n] for n in _GRAD_NAMES)
 
 
+# The leaves that RenderFunction takes as tensors: a call needs their shapes only.
+_LEAVES = ("position", "normal", "colour", "texture", "specular_map", "uv", "normal_map")
+
+
+def _host(x):
+    return x.detach().cpu().numpy() if isinstance(x, torch.Tensor) else x
+
+
+def _host_tuple(nt):
+    """The tuple with its tensors as host arrays, but for those in _LEAVES."""
+    return type(nt)(*(v.detach() if isinstance(v, torch.Tensor) and f in _LEAVES
+                      else _host_tuple(v) if hasattr(v, "_fields") else _host(v)
+                      for f, v in zip(nt._fields, nt)))
+
+
 def darboux_leaves(shader, leaf) -> tuple:
     """(uvs, normal_maps) tensors for phong_darboux, whose image depends on
     them continuously; (None, None) for the other shaders."""
@@ -147,8 +163,9 @@ def _as_tensor(x, dev) -> torch.Tensor:
 
 def _row_tensor(dev, camera, extra, call: RasterCall) -> torch.Tensor:
     """[1, 69] parameter row assembled (differentiably) from the camera and the
-    extra input's tensors, defaults from the call's scene record."""
-    base = torch.as_tensor(scene_rows(call.scenes)[0], device=dev)
+    extra input's tensors, defaults from the call's scene record; on the host
+    where none of them is a tensor."""
+    base = scene_rows(call.scenes)[0]
     parts = []
     pos = 0
     vals = {}
@@ -165,6 +182,10 @@ def _row_tensor(dev, camera, extra, call: RasterCall) -> torch.Tensor:
     shadow = getattr(extra, "shadow", None)
     if shadow is not None:
         vals["shadow_strength"] = shadow.strength
+    if not any(isinstance(v, torch.Tensor) for v in vals.values()):
+        # nothing to differentiate: the call's own record, which holds these values
+        return torch.as_tensor(base)[None, :]
+    base = torch.as_tensor(base, device=dev)
     for name, (o, n) in sorted(_SLICES.items(), key=lambda kv: kv[1][0]):
         if o > pos:
             parts.append(base[pos:o])
@@ -227,19 +248,16 @@ def render_views_differentiable(cameras: Sequence, shader, face_indices, extra, 
         raise NotImplementedError("render_views_differentiable supports the built-in shaders")
     dev = _raster.require_device()
 
-    def host(x):
-        return x.detach().cpu().numpy() if isinstance(x, torch.Tensor) else x
-
-    def host_tuple(nt):
-        return type(nt)(*(host(v) if not hasattr(v, "_fields") else host_tuple(v) for v in nt))
-
-    cams_h = [type(c)(*(host(v) for v in c)) for c in cameras]
-    extra_h = host_tuple(extra)
-    call = build_views_call(cams_h, shader, host(face_indices), extra_h, width, height,
+    cams_h = [type(c)(*(_host(v) for v in c)) for c in cameras]
+    extra_h = _host_tuple(extra)
+    call = build_views_call(cams_h, shader, _host(face_indices), extra_h, width, height,
                             init_buffers=True, zbuffer_default=zbuffer_default,
                             colour_default=colour_default)
     one = RasterCall(**{**call.__dict__, "scenes": call.scenes[:1]})
-    params = torch.cat([_row_tensor(dev, cam, extra, one) for cam in cameras])
+    rows = [_row_tensor(dev, cam, extra, one) for cam in cameras]
+    if len({r.device for r in rows}) > 1:
+        rows = [r.to(dev) for r in rows]
+    params = torch.cat(rows)
 
     def leaf(name):
         v = getattr(extra, name, None)
@@ -259,15 +277,9 @@ def render_differentiable(camera, shader, face_indices, extra, width: int, heigh
         raise NotImplementedError("render_differentiable supports the built-in shaders")
     dev = _raster.require_device()
 
-    def host(x):
-        return x.detach().cpu().numpy() if isinstance(x, torch.Tensor) else x
-
-    def host_tuple(nt):
-        return type(nt)(*(host(v) if not hasattr(v, "_fields") else host_tuple(v) for v in nt))
-
-    cam_h = type(camera)(*(host(v) for v in camera))
-    extra_h = host_tuple(extra)
-    call = build_call(cam_h, shader, host(face_indices), extra_h, width, height,
+    cam_h = type(camera)(*(_host(v) for v in camera))
+    extra_h = _host_tuple(extra)
+    call = build_call(cam_h, shader, _host(face_indices), extra_h, width, height,
                       init_buffers=True, zbuffer_default=zbuffer_default,
                       colour_default=colour_default)
     params = _row_tensor(dev, camera, extra, call)

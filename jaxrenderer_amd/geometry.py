@@ -92,9 +92,9 @@ def matmul(a: np.ndarray, b: np.ndarray) -> np.ndarray:
     squeeze = b.ndim == 1
     if squeeze:
         b = b[:, None]
-    acc = (a[:, 0:1] * b[0:1, :]).astype(f32)
+    acc = a[:, 0:1] * b[0:1, :]
     for k in range(1, a.shape[1]):
-        acc = (acc + (a[:, k : k + 1] * b[k : k + 1, :]).astype(f32)).astype(f32)
+        acc = acc + a[:, k : k + 1] * b[k : k + 1, :]
     return acc[:, 0] if squeeze else acc
 
 
@@ -139,6 +139,49 @@ def inv(a: ArrayLike) -> np.ndarray:
                     X[k, c] = f32(X[k, c] / A[k, k])
                     for i in range(k):
                         X[i, c] = f32(X[i, c] - f32(X[k, c] * A[i, k]))
+    return X
+
+
+def inv_stack(a: np.ndarray) -> np.ndarray:
+    """`inv` of each matrix of a [n, N, N] stack: its operations in its order, each on
+    all matrices at once, its conditions as selections.  A scene's 18 object
+    transforms: 0.95 ms one by one, 0.1 ms together."""
+    A = asf32(a)
+    n, N = A.shape[0], A.shape[1]
+    every = np.arange(n)
+    perm = np.tile(np.arange(N), (n, 1))
+    X = np.zeros((n, N, N), dtype=f32)
+    with np.errstate(all="ignore"):
+        for j in range(N):
+            p = np.full(n, j)
+            amax = np.abs(A[:, j, j])
+            for i in range(j + 1, N):
+                v = np.abs(A[:, i, j])
+                more = v > amax
+                amax = np.where(more, v, amax)
+                p[more] = i
+            nz = A[every, p, j] != 0
+            swap = np.nonzero(nz & (p != j))[0]
+            if swap.size:
+                q = p[swap]
+                A[swap, j], A[swap, q] = A[swap, q], A[swap, j]
+                perm[swap, j], perm[swap, q] = perm[swap, q], perm[swap, j]
+            piv = A[:, j, j, None]
+            below = A[:, j + 1:, j]
+            scaled = np.where(np.abs(piv) >= np.finfo(f32).tiny, below * (f32(1.0) / piv),
+                              below / piv)
+            A[:, j + 1:, j] = np.where(nz[:, None], scaled, below)
+            A[:, j + 1:, j + 1:] = (A[:, j + 1:, j + 1:] -
+                                    A[:, j + 1:, j, None] * A[:, None, j, j + 1:])
+        X[every[:, None], np.arange(N)[None], perm] = 1.0
+        for k in range(N - 1):
+            x = X[:, None, k]
+            X[:, k + 1:] = np.where(x != 0, X[:, k + 1:] - x * A[:, k + 1:, k, None], X[:, k + 1:])
+        for k in range(N - 1, -1, -1):
+            on = X[:, k] != 0
+            X[:, k] = np.where(on, X[:, k] / A[:, k, k, None], X[:, k])
+            x = X[:, None, k]
+            X[:, :k] = np.where(on[:, None], X[:, :k] - x * A[:, :k, k, None], X[:, :k])
     return X
 
 
@@ -224,7 +267,7 @@ class Camera(NamedTuple):
         projection = asf32(projection)
         viewport = asf32(viewport)
         view_inv = inv(view) if view_inv is None else asf32(view_inv)
-        if np.isclose(projection[3, 3], 0):
+        if abs(float(projection[3, 3])) <= 1e-8:
             projection_inv = cls.perspective_projection_matrix_inv(projection)
         else:
             projection_inv = cls.orthographic_projection_matrix_inv(projection)
@@ -259,9 +302,9 @@ class Camera(NamedTuple):
         M = asf32(matrix)
         single = p.ndim == 1
         p2 = p[None, :] if single else p
-        acc = (p2[:, 0:1] * M[None, :, 0]).astype(f32)
+        acc = p2[:, 0:1] * M[None, :, 0]
         for j in range(1, 4):
-            acc = (acc + (p2[:, j : j + 1] * M[None, :, j]).astype(f32)).astype(f32)
+            acc = acc + p2[:, j : j + 1] * M[None, :, j]
         return acc[0] if single else acc
 
     @classmethod

@@ -14,7 +14,7 @@ from typing import List, NamedTuple, Optional, Sequence, Tuple
 
 import numpy as np
 
-from .geometry import Camera, asf32, inv, transform_matrix_from_rotation
+from .geometry import _sum_sq, asf32, inv_stack, transform_matrix_from_rotation
 
 f32 = np.float32
 
@@ -114,11 +114,11 @@ class MergedModel(NamedTuple):
         dims = maps[0].ndim
         single = tuple(max(m.shape[i] for m in maps) for i in range(dims))
         dtype = np.result_type(*maps)
-        padded = [
-            np.pad(np.asarray(m), [(0, single[i] - m.shape[i]) for i in range(dims)]).astype(dtype)
-            for m in maps
-        ]
-        return np.concatenate(padded, axis=0), (single[0], single[1])
+        merged = np.zeros((len(maps) * single[0],) + single[1:], dtype=dtype)
+        for k, m in enumerate(maps):
+            at = tuple(slice(0, m.shape[i]) for i in range(1, dims))
+            merged[(slice(k * single[0], k * single[0] + m.shape[0]),) + at] = m
+        return merged, (single[0], single[1])
 
     @staticmethod
     def uv_repeat(uv, shape, map_index, offset):
@@ -177,30 +177,55 @@ def batch_models(models: Sequence[MergedModel]) -> MergedModel:
     )
 
 
+def _apply_rows(points: np.ndarray, w: np.float32, matrices: np.ndarray,
+                counts: Sequence[int]) -> np.ndarray:
+    """Camera.apply of each object's [x, y, z, w] rows and matrix, sums left to right."""
+    M = np.repeat(matrices, counts, axis=0)
+    acc = points[:, 0:1] * M[:, :, 0]
+    for j in range(1, 3):
+        acc = acc + points[:, j : j + 1] * M[:, :, j]
+    return acc + w * M[:, :, 3]
+
+
+def _normalised_parts(v: np.ndarray, counts: Sequence[int]) -> np.ndarray:
+    """geometry.normalise of each object's rows: divided by the norm of all of them."""
+    ends = np.cumsum(counts)
+    n = np.array([np.sqrt(_sum_sq(v[e - c : e])) for e, c in zip(ends, counts)], dtype=f32)
+    with np.errstate(all="ignore"):
+        return v / np.repeat(n, counts)[:, None]
+
+
 def merge_objects(objects: Sequence[ModelObject]) -> MergedModel:
     """renderer/model.py:445-555."""
     models = [o.model for o in objects]
-    counts: List[int] = [len(m.verts) for m in models]
-    map_indices = MergedModel.generate_object_vert_info(counts, list(range(len(models)))).astype(
-        np.int32
-    )
+    if not models:
+        raise ValueError("need at least one object to merge")
+    map_indices = np.repeat(np.arange(len(models), dtype=np.int32),
+                            [len(m.verts) for m in models])
     map_wh = np.asarray([m.diffuse_map.shape[:2] for m in models], dtype=np.int32)
-    double_sided = MergedModel.generate_object_vert_info(
-        counts, [bool(o.double_sided) for o in objects]
-    ).astype(bool)
+    double_sided = np.repeat(np.array([bool(o.double_sided) for o in objects]),
+                             [len(m.verts) for m in models])
     diffuse_map, single_shape = MergedModel.merge_maps([asf32(m.diffuse_map) for m in models])
     specular_map = MergedModel.merge_maps([asf32(m.specular_map) for m in models])[0]
 
-    world = [
-        Camera.apply_pos((asf32(o.model.verts) * asf32(o.local_scaling)).astype(f32), o.transform)
-        for o in objects
-    ]
-    verts, faces = MergedModel.merge_verts(world, [m.faces for m in models])
-    normals = [
-        Camera.apply_vec(asf32(o.model.norms), np.ascontiguousarray(inv(o.transform).T))
-        for o in objects
-    ]
-    norms, faces_norm = MergedModel.merge_verts(normals, [m.faces_norm for m in models])
+    # Every object's poses at once, one row of its matrix per vertex: the operations of
+    # Camera.apply_pos and Camera.apply_vec on each object, in their order
+    poses = np.stack([asf32(o.transform) for o in objects])
+    verts, faces = MergedModel.merge_verts([asf32(m.verts) for m in models],
+                                           [m.faces for m in models])
+    n_verts = [len(m.verts) for m in models]
+    scaling = np.stack([np.broadcast_to(asf32(o.local_scaling), (3,)) for o in objects])
+    verts = verts * np.repeat(scaling, n_verts, axis=0)
+    with np.errstate(all="ignore"):
+        h = _apply_rows(verts, f32(1.0), poses, n_verts)
+        verts = np.where(h[:, 3:] == 0.0, h[:, :3], h[:, :3] / h[:, 3:])
+    norms, faces_norm = MergedModel.merge_verts([asf32(m.norms) for m in models],
+                                                [m.faces_norm for m in models])
+    n_norms = [len(m.norms) for m in models]
+    norms = _normalised_parts(norms, n_norms)
+    with np.errstate(all="ignore"):
+        h = _apply_rows(norms, f32(0.0), inv_stack(poses).transpose(0, 2, 1), n_norms)
+    norms = _normalised_parts(np.ascontiguousarray(h[:, :3]), n_norms)
     uvs, faces_uv = MergedModel.merge_verts([asf32(m.uvs) for m in models],
                                             [m.faces_uv for m in models])
     return MergedModel(

@@ -164,6 +164,11 @@ typedef struct jr_frame {
   int32_t part;            /* JR_PART_ALL: every stage; JR_PART_BIN: stages 1-5 (clear,
                               setup, wide, scan, bin) only; JR_PART_RASTER: stage 6 only,
                               on a workspace holding this frame's JR_PART_BIN results */
+  int32_t keep_keys;       /* nonzero: the workspace was zeroed when it was allocated and is
+                              written to by this library only, so a pass of 2^20 pixels and
+                              more may keep its small-triangle keys in it from call to call
+                              (jr_workspace_size) instead of clearing them; the same for
+                              both parts of a split pass.  In what was the struct's padding. */
 } jr_frame;
 
 /* jr_frame.part.  Splitting a pass lets a caller overlap one pass's binning
@@ -249,7 +254,8 @@ int64_t jr_sizeof(int32_t which);
  * depth pass in the narrow form (JR_SHADER_DEPTH, init_buffers, apply_offset,
  * an offset other than -0, no prim_id / bary) keeps its small-triangle keys
  * in the workspace from call to call, each binning's tagged apart from the
- * older ones, so that it never clears them: zero a newly allocated workspace
+ * older ones, so that it never clears them (other passes do so where the frame
+ * says keep_keys): zero a newly allocated workspace
  * (memory that held a workspace of the same size before could pass for one
  * whose keys are in order), keep one workspace per stream and do not write
  * to it between calls.  A workspace used by another kind of pass in between,
@@ -278,7 +284,7 @@ int32_t jr_forward(const jr_frame* frame, const jr_inputs* inputs,
  * is never recorded.  Every call on a GPU shares that GPU's scratch: calls
  * that overlap in time on one GPU (two streams, two threads) race and must be
  * serialised by the caller.  Each call clears what it reads before writing
- * it, except the narrow form's tagged small-triangle keys (see
+ * it, except the tagged small-triangle keys (see
  * jr_workspace_size), whose older tags lose to the call's own: no result
  * depends on an earlier call. */
 #define JR_SCRATCH_BYTES (64LL << 20)

@@ -132,6 +132,7 @@ class JrFrame(ctypes.Structure):
         ("tiles_per_group", c_i32),
         ("pixels_per_lane", c_i32),
         ("part", c_i32),
+        ("keep_keys", c_i32),
     ]
 
 

@@ -168,7 +168,7 @@ def make_frame(*, width, height, n_scenes, shader, init_buffers=False, apply_off
                zbuffer_default=1.0, colour_default=(1.0, 1.0, 1.0), depth_offset=0.0,
                tile=DEFAULT_TILE, persistent=False, capacity=0,
                tiles_per_group: int = 1, pixels_per_lane: int = 1,
-               part: int = _hip.PART_ALL) -> _hip.JrFrame:
+               part: int = _hip.PART_ALL, keep_keys: bool = False) -> _hip.JrFrame:
     fr = _hip.JrFrame()
     fr.bin_capacity = int(capacity)
     fr.width, fr.height, fr.n_scenes, fr.shader = int(width), int(height), int(n_scenes), int(shader)
@@ -185,6 +185,7 @@ def make_frame(*, width, height, n_scenes, shader, init_buffers=False, apply_off
     fr.tiles_per_group = int(tiles_per_group)
     fr.pixels_per_lane = int(pixels_per_lane)
     fr.part = int(part)
+    fr.keep_keys = int(bool(keep_keys))
     return fr
 
 
@@ -223,6 +224,7 @@ def forward(
     part: int = _hip.PART_ALL,
     noalloc: bool = False,
     shadow_source: Optional["ShadowSource"] = None,
+    keep_keys: Optional[bool] = None,
 ) -> None:
     """One jr_forward call on `stream` (torch's current stream by default).
     `part`: every stage, or only the binning stages (PART_BIN) or only the
@@ -231,7 +233,8 @@ def forward(
     the library's own per-GPU scratch (no allocation at all; frames up to
     SCRATCH_BYTES of workspace, whole passes only).  `shadow_source`
     (phong_reflection_shadow): compute the shadow depths from that shadow
-    pass's binning instead of reading inputs["shadow_maps"]."""
+    pass's binning instead of reading inputs["shadow_maps"].  `keep_keys`
+    (jr_frame): by default for the workspaces that this module keeps."""
     L = _hip.lib()
     dev = zbuffer.device
     if dev.type != "cuda":
@@ -244,7 +247,9 @@ def forward(
                     zbuffer_default=zbuffer_default, colour_default=colour_default,
                     depth_offset=depth_offset, tile=tile, persistent=persistent, capacity=cap,
                     tiles_per_group=tiles_per_group, pixels_per_lane=pixels_per_lane,
-                    part=part)
+                    part=part,
+                    keep_keys=(workspace is None and not noalloc) if keep_keys is None
+                    else keep_keys)
     jin = _hip.JrInputs()
     for name, dt in _INPUT_FIELDS:
         setattr(jin, name, _ptr(inputs.get(name), name, dt, dev))

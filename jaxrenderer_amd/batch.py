@@ -213,7 +213,7 @@ class _Pass:
             zbuffer_default=c.zbuffer_default, colour_default=c.colour_default,
             depth_offset=c.depth_offset, tile=self.tile, persistent=self.persistent,
             capacity=self.capacity, tiles_per_group=self.tiles_per_group,
-            pixels_per_lane=self.pixels_per_lane, part=part)
+            pixels_per_lane=self.pixels_per_lane, part=part, keep_keys=True)
 
     def launch(self, part: int = _hip.PART_ALL, shadow_source=None) -> None:
         c = self.call
@@ -227,7 +227,7 @@ class _Pass:
             persistent=self.persistent, tiles_per_group=self.tiles_per_group,
             pixels_per_lane=self.pixels_per_lane,
             capacity=self.capacity, workspace=self.workspace, part=part,
-            shadow_source=shadow_source)
+            shadow_source=shadow_source, keep_keys=True)
 
     def pairs(self) -> int:
         c = self.call

@@ -62,6 +62,7 @@ struct Frame {
   // barycentrics) plus a nonzero offset: the small-triangle keys are 32-bit
   // depth keys kept in the zbuffer itself
   int32_t narrow;
+  int32_t tagged;  // the small-triangle keys carry their binning's tag (wide_key)
   int32_t wide_waves;  // wavefronts per wide triangle of the binning (k_wide)
   int64_t keys_at;     // offset of the key buffer in its workspace
 };

@@ -359,21 +359,30 @@ JR_DEV bool has_nan_column(const float4& r) {
   return (r.x != r.x) || (r.y != r.y) || (r.z != r.z);
 }
 
-// Small-triangle keys of the narrow form.  They live in the workspace's key
-// buffer as 64-bit words (tag << 32) | depth key, tag = ~epoch of the binning
-// that wrote them, and stay there from call to call: each binning of the
-// workspace takes the next epoch, whose smaller tag wins every atomic minimum
-// against an older word, and a word with another tag reads as "no
-// candidate".  So the buffer is not cleared per call, only when the key
-// state does not describe it: a new or foreign workspace, another pixel
-// count or buffer offset, any other binning on the workspace in between (the
-// state sits at the workspace's start, where every layout keeps it, and the
-// wide form's k_clear marks it stale), or the epoch running out.  The fill
-// value ~0 has tag 0xFFFFFFFF, which no epoch >= 1 produces.
+// Small-triangle keys live in the workspace's key buffer as 64-bit words with the tag
+// of the binning that wrote them on top, and stay there from call to call: each
+// binning of the workspace takes the next epoch, whose smaller tag wins every atomic
+// minimum against an older word, and a word with another tag reads as "no
+// candidate".  So the buffer is not cleared per call (8 bytes a pixel: 512 frames
+// of 480x270 with gradients 3,682 -> 3,511 us without it), only when the key state does not describe it: a
+// new or foreign workspace, another form, pixel count or buffer offset, any other
+// binning on the workspace in between (the state sits at the workspace's start, where
+// every layout keeps it), or the epoch running out.  The fill value ~0 has a tag that
+// no epoch >= 1 produces.
+//   narrow form: (tag << 32) | depth key, tag = ~epoch (32 bits)
+//   wide form:   (tag << 56) | depth key << 24 | id, tag = 255 - epoch (8 bits: a fill
+//                every 254 calls), where the frame says keep_keys, for up to 2^24
+//                triangles and from 2^20 pixels on;
+//                else, untagged, (depth key << 32) | id, cleared by every call
 constexpr int kKsMagic = 0, kKsPixLo = 1, kKsPixHi = 2, kKsOffLo = 3, kKsOffHi = 4,
               kKsEpoch = 5;
-constexpr uint32_t kKeyMagic = 0x6b657973u;
+constexpr uint32_t kKeyMagic = 0x6b657973u, kKeyMagicWide = 0x6b657977u;
+constexpr int32_t kTaggedTris = 1 << 24;
+constexpr int64_t kTaggedPixels = 1 << 20;
 
+JR_DEV uint64_t wide_key(uint32_t key, int32_t id, uint32_t tag) {
+  return ((uint64_t)tag << 56) | ((uint64_t)key << 24) | (uint32_t)id;
+}
 JR_DEV uint64_t tagged_key(uint32_t key, uint32_t tag) {
   return ((uint64_t)tag << 32) | key;
 }
@@ -381,7 +390,7 @@ JR_DEV uint32_t untag_key(uint64_t k, uint32_t tag) {
   return (uint32_t)(k >> 32) == tag ? (uint32_t)k : ~0u;
 }
 
-// The epoch of a narrow binning, and whether its key buffer has to be filled
+// The epoch of a tagged binning, and whether its key buffer has to be filled
 // first (then epoch 1): a function of the state that the last binning left,
 // which k_clear and k_setup each evaluate and k_offsets, after both, advances
 // (a launch of its own for that took 3 to 5 us of every call).
@@ -392,15 +401,16 @@ struct KeyEpoch {
 JR_DEV KeyEpoch next_epoch(const uint32_t* __restrict__ ks, const Frame& f) {
   const uint64_t n = (uint64_t)f.W * (uint64_t)f.H * (uint64_t)f.n_scenes, at = (uint64_t)f.keys_at;
   const uint32_t e = ks[kKsEpoch];
-  const bool ok = ks[kKsMagic] == kKeyMagic && ks[kKsPixLo] == (uint32_t)n &&
+  const bool ok = ks[kKsMagic] == (f.narrow ? kKeyMagic : kKeyMagicWide) && ks[kKsPixLo] == (uint32_t)n &&
                   ks[kKsPixHi] == (uint32_t)(n >> 32) && ks[kKsOffLo] == (uint32_t)at &&
-                  ks[kKsOffHi] == (uint32_t)(at >> 32) && e >= 1u && e < 0xFFFFFFFEu;
+                  ks[kKsOffHi] == (uint32_t)(at >> 32) && e >= 1u &&
+                  e < (f.narrow ? 0xFFFFFFFEu : 254u);
   return {ok ? e + 1u : 1u, !ok};
 }
 JR_DEV void advance_epoch(uint32_t* __restrict__ ks, const Frame& f) {
   const uint64_t n = (uint64_t)f.W * (uint64_t)f.H * (uint64_t)f.n_scenes, at = (uint64_t)f.keys_at;
   ks[kKsEpoch] = next_epoch(ks, f).epoch;
-  ks[kKsMagic] = kKeyMagic;
+  ks[kKsMagic] = f.narrow ? kKeyMagic : kKeyMagicWide;
   ks[kKsPixLo] = (uint32_t)n;
   ks[kKsPixHi] = (uint32_t)(n >> 32);
   ks[kKsOffLo] = (uint32_t)at;
@@ -408,8 +418,8 @@ JR_DEV void advance_epoch(uint32_t* __restrict__ ks, const Frame& f) {
 }
 
 // Clears the tile counters (n32 int32), sets the n64 per-pixel keys to "no
-// candidate" (the narrow form: only when next_epoch asks for a fill; the
-// wide form: always, and the key state no longer describes the buffer) and
+// candidate" (tagged keys: only when next_epoch asks for a fill; untagged ones
+// always, and the key state no longer describes the buffer) and
 // fills every scene's sample table: the NDC coordinates pix_x(i) for i < W
 // followed by pix_y(j) for j < H.
 __global__ void k_clear(int32_t* __restrict__ p32, int64_t n32, uint64_t* __restrict__ p64,
@@ -433,7 +443,7 @@ __global__ void k_clear(int32_t* __restrict__ p32, int64_t n32, uint64_t* __rest
     }
   }
   for (int64_t i = first; i < n32; i += stride) p32[i] = 0;
-  if (f.narrow) {
+  if (f.tagged) {
     if (!next_epoch(ks, f).fill) n64 = 0;
   } else if (first == 0) {
     ks[kKsMagic] = 0u;
@@ -819,7 +829,9 @@ __global__ __launch_bounds__(kSetupThreads) __attribute__((amdgpu_waves_per_eu(8
     vz1 = scenes[s_lo].viewport[11];
     __syncthreads();
   }
-  const uint32_t tag = f.narrow ? ~next_epoch(ks, f).epoch : 0u;  // this binning's key tag
+  // this binning's key tag
+  const uint32_t epoch = f.tagged ? next_epoch(ks, f).epoch : 0u;
+  const uint32_t tag = f.narrow ? ~epoch : 255u - epoch;
   // the tile raster's exact per-pixel arithmetic for every (triangle, pixel)
   auto small_pairs = [&](auto from_lds) {
     constexpr bool LDS = decltype(from_lds)::value;
@@ -855,7 +867,8 @@ __global__ __launch_bounds__(kSetupThreads) __attribute__((amdgpu_waves_per_eu(8
           atomicMin((unsigned long long*)(keys + pix), (unsigned long long)tagged_key(key, tag));
         else
           atomicMin((unsigned long long*)(keys + pix),
-                    (unsigned long long)pack_key(key, sm.u.t.tri[o]));
+                    (unsigned long long)(f.tagged ? wide_key(key, sm.u.t.tri[o], tag)
+                                                  : pack_key(key, sm.u.t.tri[o])));
       }
     }
   };
@@ -998,7 +1011,7 @@ __global__ __launch_bounds__(kOffThreads) void k_offsets(const int32_t* __restri
 #pragma unroll
     for (int w = 0; w < kOffThreads / 64; ++w) all += wave_total[w];
     first = all != 0 ? atomicAdd(total, all) : 0;
-    if (f.narrow && blockIdx.x == 0) advance_epoch(ks, f);
+    if (f.tagged && blockIdx.x == 0) advance_epoch(ks, f);
   }
   __syncthreads();
   int32_t run = first + incl - sum;
@@ -1504,7 +1517,8 @@ JR_DEV void raster_tile(const RasterArgs& a, int64_t gt, float4* lds_rec,
   // with NT a multiple of TH all of a thread's pixels share one j (and y)
   constexpr bool kOneRow = (NT % TH) == 0;
   const float* sx = a.samples + (int64_t)s * (f.W + f.H);
-  const uint32_t ktag = f.narrow ? ~a.ks[kKsEpoch] : 0u;
+  const uint32_t epoch = f.tagged ? a.ks[kKsEpoch] : 0u;
+  const uint32_t ktag = f.narrow ? ~epoch : 255u - epoch;
   // Keys are read, 8 bytes a pixel, only where a small triangle's box meets the tile:
   // half of a 480x270 frame's tiles and most of a 512x512 shadow map's have none.
   // 512 such frames with their gradients 3,959 -> 3,678 us, 60 without 191 -> 181 us.
@@ -1531,9 +1545,9 @@ JR_DEV void raster_tile(const RasterArgs& a, int64_t gt, float4* lds_rec,
         }
       } else {
         const uint64_t k0 = a.keys[pix];
-        if (k0 != ~0ull) {
-          best_key[q] = (uint32_t)(k0 >> 32);
-          best_id[q] = (int32_t)(uint32_t)k0;
+        if (f.tagged ? (uint32_t)(k0 >> 56) == ktag : k0 != ~0ull) {
+          best_key[q] = (uint32_t)(k0 >> (f.tagged ? 24 : 32));
+          best_id[q] = (int32_t)((uint32_t)k0 & (f.tagged ? kTaggedTris - 1u : ~0u));
         }
       }
     }
@@ -1756,7 +1770,7 @@ int32_t log2_exact(int32_t v) {
 
 // The kernels' view of a frame; `narrow`: the depth-only form whose
 // small-triangle keys stay in the zbuffer.
-Frame dev_frame(const jr_frame* fr, bool narrow) {
+Frame dev_frame(const jr_frame* fr, bool narrow, int32_t n_tris) {
   Frame f;
   f.W = fr->width;
   f.H = fr->height;
@@ -1772,6 +1786,10 @@ Frame dev_frame(const jr_frame* fr, bool narrow) {
   f.n_scenes = fr->n_scenes;
   f.capacity = fr->bin_capacity;
   f.narrow = narrow;
+  // (small pictures' keys are cleared in no time, and reading the epoch costs a
+  // 960x540 frame 1.5 of 74 us; 60 of 480x270 take 170 us instead of 181)
+  f.tagged = narrow || (fr->keep_keys && n_tris <= kTaggedTris &&
+                        (int64_t)f.W * f.H * f.n_scenes >= kTaggedPixels);
   f.wide_waves = wide_waves(f.T);
   f.keys_at = 0;
   return f;
@@ -2014,7 +2032,7 @@ namespace jr {
 int32_t forward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* scenes,
                      jr_outputs* out, char* ws, const WsLayout& L, hipStream_t st,
                      bool timed) {
-  Frame f = dev_frame(fr, narrow_form(fr, out->prim_id || out->bary));
+  Frame f = dev_frame(fr, narrow_form(fr, out->prim_id || out->bary), in->n_tris);
   f.keys_at = L.keys;
 
   float4* rec = reinterpret_cast<float4*>(ws + L.rec);
@@ -2049,8 +2067,8 @@ int32_t forward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* sc
   // can be graph-captured); the narrow form's tagged keys are filled only
   // when their state asks for it
   const int64_t nz = (L.offsets - L.counts) / 4;
-  // (the narrow form fills its keys only now and then: a smaller grid)
-  const int64_t nclr = std::max(std::max(nz, f.narrow ? std::min<int64_t>(L.n_pix, 1 << 20)
+  // (tagged keys are filled only now and then: a smaller grid)
+  const int64_t nclr = std::max(std::max(nz, f.tagged ? std::min<int64_t>(L.n_pix, 1 << 18)
                                                       : L.n_pix),
                                 (int64_t)(f.W + f.H) * f.n_scenes);
   hipLaunchKernelGGL(k_clear, dim3((unsigned)std::min<int64_t>((nclr + 255) / 256, 8192)),
@@ -2129,7 +2147,7 @@ int32_t forward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* sc
     a.sl.ks = reinterpret_cast<const uint32_t*>(sw + SL.kstate);
     a.sl.scenes = src.scenes;
     a.sl.texels = src.texels;
-    a.sl.f = dev_frame(src.frame, true);
+    a.sl.f = dev_frame(src.frame, true, src.n_tris);
     a.sl.zdef = src.frame->zbuffer_default;
     a.sl.depth_offset = src.frame->depth_offset;
     a.shadow_on_demand = 1;

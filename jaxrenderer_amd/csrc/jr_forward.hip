@@ -355,6 +355,11 @@ constexpr int32_t kBinListAt = 32;
 constexpr uint32_t kMaskNone = 0u;
 constexpr uint32_t kMaskWide = ~0u;
 
+// Top bit of a tile's cursor (the entries of its list that k_bin has handed out):
+// k_setup sets it in the tiles that a small triangle's pixel box meets, before k_bin
+// counts in the bits below.
+constexpr int32_t kKeyedTile = (int32_t)0x80000000u;
+
 JR_DEV bool has_nan_column(const float4& r) {
   return (r.x != r.x) || (r.y != r.y) || (r.z != r.z);
 }
@@ -733,7 +738,7 @@ __global__ __launch_bounds__(kSetupThreads) __attribute__((amdgpu_waves_per_eu(8
       const Rect kt = tiles_of(px, f);  // mostly one tile
       for (int32_t tx = kt.tx0; tx <= kt.tx1; ++tx)
         for (int32_t ty = kt.ty0; ty <= kt.ty1; ++ty)
-          keyed[(int64_t)s * f.T + tx * f.tiles_y + ty] = 1;
+          keyed[(int64_t)s * f.T + tx * f.tiles_y + ty] = kKeyedTile;
     }
     const int64_t n_t =
         (r.tx0 > r.tx1) ? 0 : (int64_t)(r.tx1 - r.tx0 + 1) * (r.ty1 - r.ty0 + 1);
@@ -943,7 +948,7 @@ JR_DEV void wide_tiles(const jr_scene* __restrict__ scenes, const Frame& f,
         if (pass) {
           const int64_t gt = tbase + tx * f.tiles_y + ty;
           if (BIN) {
-            const int64_t pos = (int64_t)offsets[gt] + atomicAdd(cursor + gt, 1);
+            const int64_t pos = (int64_t)offsets[gt] + (atomicAdd(cursor + gt, 1) & ~kKeyedTile);
             if ((uint64_t)pos < (uint64_t)f.capacity) bins[pos] = t;
           } else {
             atomicAdd(counts + gt, 1);
@@ -1089,7 +1094,7 @@ __global__ __launch_bounds__(256) void k_bin(
       const int32_t dq = div_small(q, box.z);
       const int32_t tx = box.x + dq, ty = box.y + (q - dq * box.z);
       const int64_t gt = (int64_t)box.w + tx * f.tiles_y + ty;
-      const int64_t pos = (int64_t)offsets[gt] + atomicAdd(cursor + gt, 1);
+      const int64_t pos = (int64_t)offsets[gt] + (atomicAdd(cursor + gt, 1) & ~kKeyedTile);
       if ((uint64_t)pos < (uint64_t)f.capacity) bins[pos] = own_t[o];
     }
     tile_sync<true>();  // the entries' staging is rewritten by the next step
@@ -1268,7 +1273,7 @@ struct RasterArgs {
   const int32_t* offsets;
   const int32_t* bins;
   const uint64_t* keys;
-  const int32_t* keyed;  // per tile: whether a small triangle's pixel box meets it
+  const int32_t* keyed;  // per tile: kKeyedTile where a small triangle's pixel box meets it
   const uint32_t* ks;    // key state (the narrow form's epoch)
   const float* samples;  // per scene: pix_x(i) for i < W, then pix_y(j)
   const Rect* rects;     // per-triangle tile ranges and binning words (k_setup)
@@ -1522,7 +1527,7 @@ JR_DEV void raster_tile(const RasterArgs& a, int64_t gt, float4* lds_rec,
   // Keys are read, 8 bytes a pixel, only where a small triangle's box meets the tile:
   // half of a 480x270 frame's tiles and most of a 512x512 shadow map's have none.
   // 512 such frames with their gradients 3,959 -> 3,678 us, 60 without 191 -> 181 us.
-  const bool keyed = a.keyed[gt] != 0;
+  const bool keyed = (a.keyed[gt] & kKeyedTile) != 0;
 #pragma unroll
   for (int q = 0; q < PPL; ++q) {
     const int p = tid + q * NT;
@@ -1756,7 +1761,7 @@ constexpr int64_t kAlign = 256;
 int64_t align_up(int64_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 
 struct WsLayout {
-  int64_t rec, rects, counts, cursor, keyed, offsets, misc, keys, kstate, wide, samples,
+  int64_t rec, rects, counts, cursor, offsets, misc, keys, kstate, wide, samples,
       masks, wave_scene, wbits, bins, blist, total;
   int64_t n_tiles, nblk, n_pix;
 };
@@ -1817,7 +1822,6 @@ WsLayout ws_layout(const jr_frame* fr, int32_t n_tris) {
   L.rects = o;      o += align_up(16 * (int64_t)std::max(n_tris, 1));
   L.counts = o;     o += align_up(4 * L.n_tiles);
   L.cursor = o;     o += align_up(4 * L.n_tiles);
-  L.keyed = o;      o += align_up(4 * L.n_tiles);
   L.misc = o;       o += align_up(256);  // [0] total pairs, [1] work counter, [2] wide count,
                                          // [2 + kBinListAt] k_bin's list length
   L.offsets = o;    o += align_up(4 * L.n_tiles);
@@ -2039,7 +2043,6 @@ int32_t forward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* sc
   Rect* rects = reinterpret_cast<Rect*>(ws + L.rects);
   int32_t* counts = reinterpret_cast<int32_t*>(ws + L.counts);
   int32_t* cursor = reinterpret_cast<int32_t*>(ws + L.cursor);
-  int32_t* keyed = reinterpret_cast<int32_t*>(ws + L.keyed);
   int32_t* misc = reinterpret_cast<int32_t*>(ws + L.misc);
   int32_t* offsets = reinterpret_cast<int32_t*>(ws + L.offsets);
   int32_t* bins = reinterpret_cast<int32_t*>(ws + L.bins);
@@ -2062,7 +2065,7 @@ int32_t forward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* sc
   StageTimer timer(st, timed && fr->part != JR_PART_RASTER);
   const int n_tris = in->n_tris;
   if (fr->part != JR_PART_RASTER) {
-  // counts, cursor, keyed and misc are contiguous: clear them, and the key buffer,
+  // counts, cursor and misc are contiguous: clear them, and the key buffer,
   // with one fill kernel (a kernel rather than hipMemsetAsync so the sequence
   // can be graph-captured); the narrow form's tagged keys are filled only
   // when their state asks for it
@@ -2079,7 +2082,7 @@ int32_t forward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* sc
     hipLaunchKernelGGL(k_setup, dim3((n_tris + kSetupThreads - 1) / kSetupThreads),
                        dim3(kSetupThreads), 0, st, *in,
                        scenes, f, rec, rects, counts, keys, wide, wide_count, samples, kstate,
-                       masks, wave_scene, blist, keyed);
+                       masks, wave_scene, blist, cursor);
   timer.mark(2);
   if (n_tris > 0)
     hipLaunchKernelGGL(k_wide, dim3(wide_groups), dim3(256), 0, st, scenes, f, rec, rects, wide,
@@ -2115,7 +2118,7 @@ int32_t forward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* sc
   a.rects = rects;
   a.masks = masks;
   a.keys = keys;
-  a.keyed = keyed;
+  a.keyed = cursor;
   a.ks = kstate;
   a.samples = samples;
   a.work_counter = misc + 1;

@@ -19,8 +19,9 @@
 //   k_bwd_prepare / k_bwd_fill  check the workspace header; clear the
 //                 per-triangle flags and accumulators only for a workspace that
 //                 no earlier call left zero (each call clears what it used)
-//   k_bwd_pixels  one wavefront per 16x16 tile (4 pixels per lane): each
-//                 distinct primitive's setup and corner stage once, in LDS;
+//   k_bwd_pixels  one wavefront per 16x16 tile (4 pixels per lane) or 8x16
+//                 tile (2; the rule is in backward_body): each distinct
+//                 primitive's setup and corner stage once, in LDS;
 //                 per pixel, shading backward (texture / specular gradients
 //                 summed per texel in LDS), the visibility backward (dL/dM^-1,
 //                 dL/dz_clip, per-corner varying cotangents) summed per

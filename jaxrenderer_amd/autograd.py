@@ -161,11 +161,11 @@ def _as_tensor(x, dev) -> torch.Tensor:
     return torch.as_tensor(np.asarray(x, dtype=np.float32), device=dev)
 
 
-def _row_tensor(dev, camera, extra, call: RasterCall) -> torch.Tensor:
+def _row_tensor(dev, camera, extra, scene: _hip.JrScene) -> torch.Tensor:
     """[1, 69] parameter row assembled (differentiably) from the camera and the
-    extra input's tensors, defaults from the call's scene record; on the host
-    where none of them is a tensor."""
-    base = scene_rows(call.scenes)[0]
+    extra input's tensors, defaults from `scene`, the record that was built from
+    them; on the host where none of them is a tensor."""
+    base = scene_rows([scene])[0]
     parts = []
     pos = 0
     vals = {}
@@ -183,7 +183,7 @@ def _row_tensor(dev, camera, extra, call: RasterCall) -> torch.Tensor:
     if shadow is not None:
         vals["shadow_strength"] = shadow.strength
     if not any(isinstance(v, torch.Tensor) for v in vals.values()):
-        # nothing to differentiate: the call's own record, which holds these values
+        # nothing to differentiate: the record holds these values
         return torch.as_tensor(base)[None, :]
     base = torch.as_tensor(base, device=dev)
     for name, (o, n) in sorted(_SLICES.items(), key=lambda kv: kv[1][0]):
@@ -253,8 +253,8 @@ def render_views_differentiable(cameras: Sequence, shader, face_indices, extra, 
     call = build_views_call(cams_h, shader, _host(face_indices), extra_h, width, height,
                             init_buffers=True, zbuffer_default=zbuffer_default,
                             colour_default=colour_default)
-    one = RasterCall(**{**call.__dict__, "scenes": call.scenes[:1]})
-    rows = [_row_tensor(dev, cam, extra, one) for cam in cameras]
+    # each view's own record: where its camera is not a tensor, the row is the record's
+    rows = [_row_tensor(dev, cam, extra, scene) for cam, scene in zip(cameras, call.scenes)]
     if len({r.device for r in rows}) > 1:
         rows = [r.to(dev) for r in rows]
     params = torch.cat(rows)
@@ -282,7 +282,7 @@ def render_differentiable(camera, shader, face_indices, extra, width: int, heigh
     call = build_call(cam_h, shader, _host(face_indices), extra_h, width, height,
                       init_buffers=True, zbuffer_default=zbuffer_default,
                       colour_default=colour_default)
-    params = _row_tensor(dev, camera, extra, call)
+    params = _row_tensor(dev, camera, extra, call.scenes[0])
 
     def leaf(name):
         v = getattr(extra, name, None)

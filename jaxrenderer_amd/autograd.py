@@ -87,7 +87,13 @@ class RenderFunction(torch.autograd.Function):
             if t is not None:
                 inputs[name] = t.detach().float().contiguous()
             elif name in ("uvs", "normal_maps") and name in call.inputs:
-                inputs[name] = _plan.to_device(call.inputs[name], dev, name)
+                given = call.inputs[name]
+                own = _plan.to_device(given, dev, name)
+                # the backward reads it again, outside torch's saved tensors: never the
+                # caller's memory, which may be written to in between
+                if isinstance(given, torch.Tensor) and own.data_ptr() == given.data_ptr():
+                    own = own.clone()
+                inputs[name] = own
             else:
                 inputs[name] = None
         B, W, H = call.n_scenes, call.width, call.height

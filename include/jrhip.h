@@ -163,12 +163,8 @@ typedef struct jr_frame {
                               tiles (one wavefront per tile) */
   int32_t part;            /* JR_PART_ALL: every stage; JR_PART_BIN: stages 1-5 (clear,
                               setup, wide, scan, bin) only; JR_PART_RASTER: stage 6 only,
-                              on a workspace holding this frame's JR_PART_BIN results */
-  int32_t keep_keys;       /* nonzero: the workspace was zeroed when it was allocated and is
-                              written to by this library only, so a pass of 2^20 pixels and
-                              more may keep its small-triangle keys in it from call to call
-                              (jr_workspace_size) instead of clearing them; the same for
-                              both parts of a split pass.  In what was the struct's padding. */
+                              on a workspace holding this frame's JR_PART_BIN results;
+                              each with JR_PART_KEEP_KEYS added where it holds */
 } jr_frame;
 
 /* jr_frame.part.  Splitting a pass lets a caller overlap one pass's binning
@@ -177,7 +173,13 @@ typedef struct jr_frame {
 enum {
   JR_PART_ALL = 0,
   JR_PART_BIN = 1,
-  JR_PART_RASTER = 2
+  JR_PART_RASTER = 2,
+  /* The workspace was zeroed when it was allocated and is written to by this library
+   * only, so a pass of 2^20 pixels and more may keep its small-triangle keys in it from
+   * call to call (jr_workspace_size) instead of clearing them.  The same for both parts
+   * of a split pass.  (A flag here, not a field of its own: in what was padding, a field
+   * would read whatever a caller that does not know it left there.) */
+  JR_PART_KEEP_KEYS = 256
 };
 
 /* Shadow depths on demand.  The shadow-map pass of renderer/shadow.py:40-125
@@ -254,8 +256,8 @@ int64_t jr_sizeof(int32_t which);
  * depth pass in the narrow form (JR_SHADER_DEPTH, init_buffers, apply_offset,
  * an offset other than -0, no prim_id / bary) keeps its small-triangle keys
  * in the workspace from call to call, each binning's tagged apart from the
- * older ones, so that it never clears them (other passes do so where the frame
- * says keep_keys): zero a newly allocated workspace
+ * older ones, so that it never clears them (other passes do so where frame->part
+ * says JR_PART_KEEP_KEYS): zero a newly allocated workspace
  * (memory that held a workspace of the same size before could pass for one
  * whose keys are in order), keep one workspace per stream and do not write
  * to it between calls.  A workspace used by another kind of pass in between,
@@ -280,7 +282,7 @@ int32_t jr_forward(const jr_frame* frame, const jr_inputs* inputs,
  * workspace is the library's own per-GPU scratch array of JR_SCRATCH_BYTES,
  * resident from the library's load to the end of the process; a frame whose
  * jr_workspace_size exceeds it is rejected with JR_E_WORKSPACE before any
- * launch.  Whole passes only (frame->part must be JR_PART_ALL); stage timing
+ * launch.  Whole passes only (JR_PART_ALL, JR_PART_KEEP_KEYS or not); stage timing
  * is never recorded.  Every call on a GPU shares that GPU's scratch: calls
  * that overlap in time on one GPU (two streams, two threads) race and must be
  * serialised by the caller.  Each call clears what it reads before writing

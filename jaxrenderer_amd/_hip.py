@@ -34,6 +34,7 @@ SHADER_VISIBILITY = 7
 STAGE_NAMES = ("clear", "setup", "wide", "scan", "bin", "raster")
 # jr_frame.part: every stage, the binning stages 1-5 only, the raster only
 PART_ALL, PART_BIN, PART_RASTER = 0, 1, 2
+PART_KEEP_KEYS = 256  # added to it: the workspace's keys may stay from call to call
 STAGES = len(STAGE_NAMES)
 
 c_f = ctypes.c_float
@@ -132,7 +133,6 @@ class JrFrame(ctypes.Structure):
         ("tiles_per_group", c_i32),
         ("pixels_per_lane", c_i32),
         ("part", c_i32),
-        ("keep_keys", c_i32),
     ]
 
 

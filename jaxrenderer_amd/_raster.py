@@ -184,8 +184,7 @@ def make_frame(*, width, height, n_scenes, shader, init_buffers=False, apply_off
     fr.persistent = int(bool(persistent))
     fr.tiles_per_group = int(tiles_per_group)
     fr.pixels_per_lane = int(pixels_per_lane)
-    fr.part = int(part)
-    fr.keep_keys = int(bool(keep_keys))
+    fr.part = int(part) | (_hip.PART_KEEP_KEYS if keep_keys else 0)
     return fr
 
 
@@ -234,7 +233,7 @@ def forward(
     SCRATCH_BYTES of workspace, whole passes only).  `shadow_source`
     (phong_reflection_shadow): compute the shadow depths from that shadow
     pass's binning instead of reading inputs["shadow_maps"].  `keep_keys`
-    (jr_frame): by default for the workspaces that this module keeps."""
+    (JR_PART_KEEP_KEYS): by default for the workspaces that this module keeps."""
     L = _hip.lib()
     dev = zbuffer.device
     if dev.type != "cuda":

@@ -376,7 +376,7 @@ JR_DEV bool has_nan_column(const float4& r) {
 // no epoch >= 1 produces.
 //   narrow form: (tag << 32) | depth key, tag = ~epoch (32 bits)
 //   wide form:   (tag << 56) | depth key << 24 | id, tag = 255 - epoch (8 bits: a fill
-//                every 254 calls), where the frame says keep_keys, for up to 2^24
+//                every 254 calls), where the frame says JR_PART_KEEP_KEYS, for up to 2^24
 //                triangles and from 2^20 pixels on;
 //                else, untagged, (depth key << 32) | id, cleared by every call
 constexpr int kKsMagic = 0, kKsPixLo = 1, kKsPixHi = 2, kKsOffLo = 3, kKsOffHi = 4,
@@ -1274,7 +1274,7 @@ struct RasterArgs {
   const int32_t* bins;
   const uint64_t* keys;
   const int32_t* keyed;  // per tile: kKeyedTile where a small triangle's pixel box meets it
-  const uint32_t* ks;    // key state (the narrow form's epoch)
+  const uint32_t* ks;    // key state (the epoch of tagged keys)
   const float* samples;  // per scene: pix_x(i) for i < W, then pix_y(j)
   const Rect* rects;     // per-triangle tile ranges and binning words (k_setup)
   const uint32_t* masks;
@@ -1767,6 +1767,9 @@ struct WsLayout {
 };
 
 
+// A frame's stages, without the flag that may come with them.
+int32_t part_of(const jr_frame* fr) { return fr->part & ~JR_PART_KEEP_KEYS; }
+
 int32_t log2_exact(int32_t v) {
   int32_t l = 0;
   while ((1 << l) < v) ++l;
@@ -1793,7 +1796,7 @@ Frame dev_frame(const jr_frame* fr, bool narrow, int32_t n_tris) {
   f.narrow = narrow;
   // (small pictures' keys are cleared in no time, and reading the epoch costs a
   // 960x540 frame 1.5 of 74 us; 60 of 480x270 take 170 us instead of 181)
-  f.tagged = narrow || (fr->keep_keys && n_tris <= kTaggedTris &&
+  f.tagged = narrow || ((fr->part & JR_PART_KEEP_KEYS) && n_tris <= kTaggedTris &&
                         (int64_t)f.W * f.H * f.n_scenes >= kTaggedPixels);
   f.wide_waves = wide_waves(f.T);
   f.keys_at = 0;
@@ -1856,8 +1859,10 @@ int32_t check_frame(const jr_frame* fr) {
     return fail(JR_E_INVALID, "2^22 or more tiles per scene");
   if (fr->bin_capacity < 0 || fr->bin_capacity > 0x7FFFFFFFLL)
     return fail(JR_E_INVALID, "bin_capacity out of range");
-  if (fr->part != JR_PART_ALL && fr->part != JR_PART_BIN && fr->part != JR_PART_RASTER)
-    return fail(JR_E_INVALID, "part must be JR_PART_ALL, JR_PART_BIN or JR_PART_RASTER");
+  const int32_t part = part_of(fr);
+  if (part != JR_PART_ALL && part != JR_PART_BIN && part != JR_PART_RASTER)
+    return fail(JR_E_INVALID, "part must be JR_PART_ALL, JR_PART_BIN or JR_PART_RASTER, each "
+                              "with or without JR_PART_KEEP_KEYS");
   if (fr->tiles_per_group < 0 || fr->tiles_per_group > 64)
     return fail(JR_E_INVALID, "tiles_per_group must be in [0, 64]");
   const bool ok_ppl = fr->pixels_per_lane <= 1 ||
@@ -2062,9 +2067,10 @@ int32_t forward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* sc
       (unsigned)std::min<int64_t>(((int64_t)in->n_tris * f.wide_waves + 3) / 4, 8192);
 
   // a binning-only call is timed too (its raster stage then takes no time)
-  StageTimer timer(st, timed && fr->part != JR_PART_RASTER);
+  const int32_t part = part_of(fr);
+  StageTimer timer(st, timed && part != JR_PART_RASTER);
   const int n_tris = in->n_tris;
-  if (fr->part != JR_PART_RASTER) {
+  if (part != JR_PART_RASTER) {
   // counts, cursor and misc are contiguous: clear them, and the key buffer,
   // with one fill kernel (a kernel rather than hipMemsetAsync so the sequence
   // can be graph-captured); the narrow form's tagged keys are filled only
@@ -2099,7 +2105,7 @@ int32_t forward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* sc
   }
   timer.mark(5);
   }
-  if (fr->part == JR_PART_BIN) {
+  if (part == JR_PART_BIN) {
     timer.mark(6);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess)
@@ -2224,7 +2230,7 @@ int32_t jr_forward_noalloc(const jr_frame* fr, const jr_inputs* in, const jr_sce
   rc = check_inputs(fr, in, out);
   if (rc) return rc;
   if (!scenes) return fail(JR_E_INVALID, "scenes is NULL");
-  if (fr->part != JR_PART_ALL)
+  if (part_of(fr) != JR_PART_ALL)
     return fail(JR_E_INVALID, "jr_forward_noalloc runs whole passes only (part = JR_PART_ALL)");
   const WsLayout L = ws_layout(fr, in->n_tris);
   if (L.total > (int64_t)JR_SCRATCH_BYTES)

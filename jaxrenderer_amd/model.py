@@ -211,11 +211,10 @@ def merge_objects(objects: Sequence[ModelObject]) -> MergedModel:
     # Every object's poses at once, one row of its matrix per vertex: the operations of
     # Camera.apply_pos and Camera.apply_vec on each object, in their order
     poses = np.stack([asf32(o.transform) for o in objects])
-    verts, faces = MergedModel.merge_verts([asf32(m.verts) for m in models],
-                                           [m.faces for m in models])
-    n_verts = [len(m.verts) for m in models]
-    scaling = np.stack([np.broadcast_to(asf32(o.local_scaling), (3,)) for o in objects])
-    verts = verts * np.repeat(scaling, n_verts, axis=0)
+    # local_scaling broadcasts against the vertices: one factor, one per axis or per vertex
+    scaled = [asf32(o.model.verts) * asf32(o.local_scaling) for o in objects]
+    verts, faces = MergedModel.merge_verts(scaled, [m.faces for m in models])
+    n_verts = [len(v) for v in scaled]
     with np.errstate(all="ignore"):
         h = _apply_rows(verts, f32(1.0), poses, n_verts)
         verts = np.where(h[:, 3:] == 0.0, h[:, :3], h[:, :3] / h[:, 3:])

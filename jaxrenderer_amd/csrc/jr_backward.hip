@@ -1499,12 +1499,14 @@ int32_t backward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* s
   a.n_scenes = fr->n_scenes;
   // Four pixels per lane (16 x 16 tiles) or two (8 x 16).  Two halve a wavefront's
   // chain of lookups and its triangles, for half as many pixels to pay for them: the
-  // faster one where the wavefronts of four are few rounds of the 4,096 that the
-  // chip holds and a tile has triangles to set up (23 views of 201x187, 3,600 such
-  // wavefronts, 190 -> 167 us; 64 of 256x256, 16,000, 411 -> 381 us; 256 scenes of
-  // 128x128 790 -> 759 us), but not where the picture is larger (512 of 480x270,
-  // 261,000 wavefronts, 4,100 against 4,480 us; 1,024 of 84x84, 29,000, 1,399 against
-  // 1,428 us) or its triangles are (64 views of a 200-triangle ball 258 against 274).
+  // faster one where the 16 x 16 tiles, partial ones included, are few rounds of the
+  // 4,096 wavefronts that the chip holds and a tile has triangles to set up (23 views
+  // of 201x187, 3,588 tiles, 190 -> 167 us; 64 of 256x256 and 256 scenes of 128x128,
+  // 16,384 each, 411 -> 381 and 790 -> 759 us), but not where there are more (1,024 of
+  // 84x84, 36,864 tiles packed into 28,672 wavefronts, 1,399 against 1,428 us; 512 of
+  // 480x270, 261,120, 4,100 against 4,480 us) or the triangles are larger (64 views of a
+  // 200-triangle ball 258 against 274).  The line is six rounds of tiles, between the
+  // largest measured gain and the smallest measured loss.
   const int64_t tiles4 = (int64_t)((a.W + 15) / 16) * ((a.H + 15) / 16) * a.n_scenes;
   const int ppl = !d_zbuffer && tiles4 <= 24576 && in->n_tris >= 4 * tiles4 ? 2 : 4;
   const int64_t QW = (a.W + ppl / 2 - 1) / (ppl / 2), QH = (a.H + 1) / 2, nq = QW * QH;

@@ -59,8 +59,8 @@ struct Frame {
   int32_t n_scenes;
   int64_t capacity;
   // depth-only pass whose output is the depth alone (no primitive ids or
-  // barycentrics) plus a nonzero offset: the small-triangle keys are 32-bit
-  // depth keys kept in the zbuffer itself
+  // barycentrics) plus an offset: the small-triangle keys are tagged 32-bit depth
+  // keys without an id
   int32_t narrow;
   int32_t tagged;  // the small-triangle keys carry their binning's tag (wide_key)
   int32_t wide_waves;  // wavefronts per wide triangle of the binning (k_wide)

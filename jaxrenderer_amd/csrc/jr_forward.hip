@@ -369,11 +369,12 @@ JR_DEV bool has_nan_column(const float4& r) {
 // binning of the workspace takes the next epoch, whose smaller tag wins every atomic
 // minimum against an older word, and a word with another tag reads as "no
 // candidate".  So the buffer is not cleared per call (8 bytes a pixel: 512 frames
-// of 480x270 with gradients 3,682 -> 3,511 us without it), only when the key state does not describe it: a
-// new or foreign workspace, another form, pixel count or buffer offset, any other
-// binning on the workspace in between (the state sits at the workspace's start, where
-// every layout keeps it), or the epoch running out.  The fill value ~0 has a tag that
-// no epoch >= 1 produces.
+// of 480x270 with gradients 3,700 -> 3,533 us without it, 60 frames 177 -> 168 us, 1,024
+// of 84x84 613 -> 602 us), only when the key state does not describe it: a new or
+// foreign workspace, another form, pixel count or buffer offset, any other binning on
+// the workspace in between (the state sits at the workspace's start, where every layout
+// keeps it), or the epoch running out.  The fill value ~0 has a tag that no epoch >= 1
+// produces.
 //   narrow form: (tag << 32) | depth key, tag = ~epoch (32 bits)
 //   wide form:   (tag << 56) | depth key << 24 | id, tag = 255 - epoch (8 bits: a fill
 //                every 254 calls), where the frame says JR_PART_KEEP_KEYS, for up to 2^24
@@ -1526,7 +1527,7 @@ JR_DEV void raster_tile(const RasterArgs& a, int64_t gt, float4* lds_rec,
   const uint32_t ktag = f.narrow ? ~epoch : 255u - epoch;
   // Keys are read, 8 bytes a pixel, only where a small triangle's box meets the tile:
   // half of a 480x270 frame's tiles and most of a 512x512 shadow map's have none.
-  // 512 such frames with their gradients 3,959 -> 3,678 us, 60 without 191 -> 181 us.
+  // 512 such frames with their gradients 3,948 -> 3,700 us, 60 without 184 -> 177 us.
   const bool keyed = (a.keyed[gt] & kKeyedTile) != 0;
 #pragma unroll
   for (int q = 0; q < PPL; ++q) {
@@ -1776,8 +1777,7 @@ int32_t log2_exact(int32_t v) {
   return l;
 }
 
-// The kernels' view of a frame; `narrow`: the depth-only form whose
-// small-triangle keys stay in the zbuffer.
+// The kernels' view of a frame; `narrow`: narrow_form().
 Frame dev_frame(const jr_frame* fr, bool narrow, int32_t n_tris) {
   Frame f;
   f.W = fr->width;
@@ -1794,8 +1794,9 @@ Frame dev_frame(const jr_frame* fr, bool narrow, int32_t n_tris) {
   f.n_scenes = fr->n_scenes;
   f.capacity = fr->bin_capacity;
   f.narrow = narrow;
-  // (small pictures' keys are cleared in no time, and reading the epoch costs a
-  // 960x540 frame 1.5 of 74 us; 60 of 480x270 take 170 us instead of 181)
+  // (fewer pixels' keys are cleared in no time, and reading the epoch costs a 960x540
+  // frame 0.9 of 83.4 us; 1.4M pixels, 200 walkers, take 154 us either way; 7.2M, 1,024
+  // frames of 84x84, 602 us instead of 613; 7.8M, 60 of 480x270, 168 instead of 179)
   f.tagged = narrow || ((fr->part & JR_PART_KEEP_KEYS) && n_tris <= kTaggedTris &&
                         (int64_t)f.W * f.H * f.n_scenes >= kTaggedPixels);
   f.wide_waves = wide_waves(f.T);
@@ -1803,9 +1804,9 @@ Frame dev_frame(const jr_frame* fr, bool narrow, int32_t n_tris) {
   return f;
 }
 
-// A depth pass with an offset and no id outputs keeps 32-bit depth keys in
-// its zbuffer (an offset of -0 would keep the sign of a -0 depth, which a key
-// cannot tell apart).
+// A depth pass with an offset and no id outputs: its small-triangle keys are tagged
+// 32-bit depth keys without an id (an offset of -0 would keep the sign of a -0 depth,
+// which a key cannot tell apart).
 bool narrow_form(const jr_frame* fr, bool ids) {
   uint32_t ob;
   std::memcpy(&ob, &fr->depth_offset, 4);
@@ -2073,10 +2074,11 @@ int32_t forward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* sc
   if (part != JR_PART_RASTER) {
   // counts, cursor and misc are contiguous: clear them, and the key buffer,
   // with one fill kernel (a kernel rather than hipMemsetAsync so the sequence
-  // can be graph-captured); the narrow form's tagged keys are filled only
-  // when their state asks for it
+  // can be graph-captured); tagged keys are filled only when their state asks for it
   const int64_t nz = (L.offsets - L.counts) / 4;
-  // (tagged keys are filled only now and then: a smaller grid)
+  // (tagged keys are filled only now and then: a smaller grid, 0.5 to 2 us shorter
+  // where there is nothing to fill, and as fast as one of 2^20 or 2^21 threads where there
+  // is: 67M pixels 95 against 101 us, 134M 196 against 194 to 205)
   const int64_t nclr = std::max(std::max(nz, f.tagged ? std::min<int64_t>(L.n_pix, 1 << 18)
                                                       : L.n_pix),
                                 (int64_t)(f.W + f.H) * f.n_scenes);

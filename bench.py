@@ -13,8 +13,10 @@ from __future__ import annotations
 
 import argparse
 import ctypes
+import hashlib
 import json
 import os
+import re
 import sys
 import time
 
@@ -115,6 +117,27 @@ def complexity_sample(scenes, width: int, height: int, smspec, n: int) -> dict:
 
 def log(msg: str) -> None:
     print(f"[bench] {msg}", file=sys.stderr, flush=True)
+
+
+def forward_source() -> str:
+    """A digest of the forward kernels' sources without their comments and spaces: which
+    kernels a committed profile was taken from."""
+    h = hashlib.sha256()
+    for name in ("jr_common.h", "jr_forward.hip", "jr_math.h", "jr_shade.h"):
+        with open(os.path.join(ROOT, "jaxrenderer_amd", "csrc", name)) as f:
+            text = re.sub(r"/\*.*?\*/", "", f.read(), flags=re.S)
+        h.update(re.sub(r"\s+", "", re.sub(r"//[^\n]*", "", text)).encode())
+    return h.hexdigest()[:16]
+
+
+def profiled() -> dict:
+    """profiles/config3_traffic.json where it was taken from these kernels, else {}."""
+    path = os.path.join(ROOT, "profiles", "config3_traffic.json")
+    if not os.path.exists(path):
+        return {}
+    with open(path) as f:
+        prof = json.load(f)
+    return prof if prof.get("source") == forward_source() else {}
 
 
 def stage_times(n_calls: int):
@@ -401,14 +424,14 @@ def main() -> None:
 
     # the implementation's own byte model per stage (what the kernels must
     # move as built: key buffers, records, lists), beside the algorithmic
-    # bytes.  The shadow pass keeps 32-bit depth keys in its output buffer
-    # (a depth pass with an offset and no id outputs); the main pass 64-bit
-    # keys.
-    key_b = {"shadow": 4, "main": 8}
+    # bytes.  Small-triangle keys are 8 bytes a pixel; tagged ones (the shadow
+    # pass's, and the main pass's from 2^20 pixels on) are not cleared.
+    key_b = {"shadow": 8, "main": 8}
+    tagged = {"shadow": True, "main": px["main"] >= 1 << 20}
 
     def impl_bytes(pass_: str, stage: str) -> int:
-        if stage == "clear":  # key per pixel, tile counters
-            return px[pass_] * key_b[pass_] + tiles[pass_] * 8
+        if stage == "clear":  # untagged keys, tile counters
+            return (0 if tagged[pass_] else px[pass_] * key_b[pass_]) + tiles[pass_] * 8
         if stage == "setup":  # 3 slot ids (+3 position indices in the main
             # pass) and 3 positions read, one 4 B binning word written per
             # triangle (records of the triangles that survive culling not
@@ -420,7 +443,8 @@ def main() -> None:
             return tiles[pass_] * 8
         if stage == "bin":  # binning word per triangle, 4 B per binned pair
             return n_tri * 4 + pairs[pass_] * 4
-        # raster: keys read, depth (+ colour) written, 52 B per binned pair
+        # raster: keys read (at most: only in tiles that a small triangle
+        # meets), depth (+ colour) written, 52 B per binned pair
         # (id + 48 B record), and per visible triangle of the main pass its
         # record (64 B), face row (12 B) and three corners' indices and
         # attributes (4 x 4 B indices + position, normal, uv: 48 B each)
@@ -437,23 +461,20 @@ def main() -> None:
         dom_fr = fractions(wm["bytes"].get(dom, 0), wm["ops"].get(dom, 0), stages[dom])
         frame_fr = fractions(wm["bytes_total"], wm["ops_total"], t_batched * 1e3)
     traffic = valu_busy = prof_tile = None
-    tpath = os.path.join(ROOT, "profiles", "config3_traffic.json")
-    if os.path.exists(tpath):
-        with open(tpath) as f:
-            prof = json.load(f)
-        measured = prof.get("kernels", {})
-        if dom in measured:
-            traffic = measured[dom]["hbm_bytes"]
-            valu_busy = measured[dom].get("valu_busy")
-            prof_tile = measured[dom].get("tile", prof.get("tile"))
-            run_p = br.passes.get(dom.split(".")[0])
-            if isinstance(prof_tile, dict) and run_p is not None:
-                same = (list(prof_tile.get("tile", [])) == list(run_p.tile)
-                        and prof_tile.get("persistent") == run_p.persistent
-                        and prof_tile.get("tiles_per_group") == run_p.tiles_per_group
-                        and prof_tile.get("pixels_per_lane") == run_p.pixels_per_lane)
-                prof_tile = (f"profiled launch {prof_tile}: "
-                             f"{'the same as' if same else 'differs from'} this run's")
+    prof = profiled()
+    measured = prof.get("kernels", {})
+    if dom in measured:
+        traffic = measured[dom]["hbm_bytes"]
+        valu_busy = measured[dom].get("valu_busy")
+        prof_tile = measured[dom].get("tile", prof.get("tile"))
+        run_p = br.passes.get(dom.split(".")[0])
+        if isinstance(prof_tile, dict) and run_p is not None:
+            same = (list(prof_tile.get("tile", [])) == list(run_p.tile)
+                    and prof_tile.get("persistent") == run_p.persistent
+                    and prof_tile.get("tiles_per_group") == run_p.tiles_per_group
+                    and prof_tile.get("pixels_per_lane") == run_p.pixels_per_lane)
+            prof_tile = (f"profiled launch {prof_tile}: "
+                         f"{'the same as' if same else 'differs from'} this run's")
     if dom_fr is not None:
         best = dom_fr[dom_fr["bound"]]
         roofline = {"bound": dom_fr["bound"], "achieved": best["achieved"], "peak": best["peak"],

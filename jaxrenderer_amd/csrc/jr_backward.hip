@@ -617,7 +617,10 @@ JR_DEV KernArgs<T> kernel_args() {
 // added, 1,758 us.  1,024 frames of 84x84: 573, 590, 538 us.
 //
 // 16 workgroups' LDS on a CU, 4 wavefronts per SIMD as 128 registers allow, takes
-// at most 10 KiB each.
+// at most 10 KiB each.  With a depth gradient the reflection shaders' three more sums
+// and six more values per pixel do not fit 128 registers (22 and 41 of them were spilt,
+// and 1,024 frames of 84x84 took 888 us): those two instances run 3 wavefronts of 168
+// (804 us).
 constexpr int tri_cap(int shader) {
   return shader == JR_SHADER_PHONG_REFLECTION_SHADOW || shader == JR_SHADER_PHONG_DARBOUX ? 28
                                                                                          : 32;
@@ -635,9 +638,13 @@ constexpr int kSearched = 12;
 constexpr int kTexShared = 16, kTexSearched = 4;
 constexpr int kMapCap = 32;  // entries of a second map (normal map, specular map)
 
+constexpr int pixel_waves(int shader, bool dz) {
+  return shader == JR_SHADER_PHONG_DARBOUX ? 2 : dz && reflects(shader) ? 3 : 4;
+}
+
 template <int SHADER, bool DZ, int PPL>
 __global__ __launch_bounds__(64)
-__attribute__((amdgpu_waves_per_eu(SHADER == JR_SHADER_PHONG_DARBOUX ? 2 : 4, 8)))
+__attribute__((amdgpu_waves_per_eu(pixel_waves(SHADER, DZ), 8)))
 void k_bwd_pixels(BwdArgs) {
   constexpr int BW = PPL / 2;  // a lane's block is BW x 2 pixels
   constexpr int kShared = shared_from(PPL);
@@ -1400,8 +1407,10 @@ template <int SHADER>
 void launch_bwd(const BwdArgs& a, int ppl, hipStream_t st) {
   const int64_t n_waves = (int64_t)a.T * a.n_scenes;
   const dim3 grid((unsigned)n_waves);
-  if (a.d_zbuffer)
+  if (a.d_zbuffer && ppl == 4)
     hipLaunchKernelGGL((k_bwd_pixels<SHADER, true, 4>), grid, dim3(64), 0, st, a);
+  else if (a.d_zbuffer)
+    hipLaunchKernelGGL((k_bwd_pixels<SHADER, true, 2>), grid, dim3(64), 0, st, a);
   else if (ppl == 4)
     hipLaunchKernelGGL((k_bwd_pixels<SHADER, false, 4>), grid, dim3(64), 0, st, a);
   else
@@ -1506,9 +1515,11 @@ int32_t backward_body(const jr_frame* fr, const jr_inputs* in, const jr_scene* s
   // 84x84, 36,864 tiles packed into 28,672 wavefronts, 1,399 against 1,428 us; 512 of
   // 480x270, 261,120, 4,100 against 4,480 us) or the triangles are larger (64 views of a
   // 200-triangle ball 258 against 274).  The line is six rounds of tiles, between the
-  // largest measured gain and the smallest measured loss.
+  // largest measured gain and the smallest measured loss.  With a depth gradient, the
+  // backward alone: 16 scenes of 100x75 139 -> 99 us, 256 of 84x84 311 -> 251, 64 phong
+  // views of 256x256 297 -> 250, 4 of 128x128 108 -> 68.
   const int64_t tiles4 = (int64_t)((a.W + 15) / 16) * ((a.H + 15) / 16) * a.n_scenes;
-  const int ppl = !d_zbuffer && tiles4 <= 24576 && in->n_tris >= 4 * tiles4 ? 2 : 4;
+  const int ppl = tiles4 <= 24576 && in->n_tris >= 4 * tiles4 ? 2 : 4;
   const int64_t QW = (a.W + ppl / 2 - 1) / (ppl / 2), QH = (a.H + 1) / 2, nq = QW * QH;
   const int64_t tiles_y = (QH + 7) / 8, tiles = (QW + 7) / 8 * tiles_y;
   // the leftover blocks are packed where that saves at least an eighth of the

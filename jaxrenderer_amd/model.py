@@ -112,6 +112,8 @@ class MergedModel(NamedTuple):
         """Pad every map with zeros to the largest extent of each axis and
         concatenate along axis 0 (renderer/model.py:249-301)."""
         dims = maps[0].ndim
+        if any(m.ndim != dims for m in maps):  # numpy would drop leading axes of 1
+            raise ValueError("maps to merge must have the same number of axes")
         single = tuple(max(m.shape[i] for m in maps) for i in range(dims))
         dtype = np.result_type(*maps)
         merged = np.zeros((len(maps) * single[0],) + single[1:], dtype=dtype)

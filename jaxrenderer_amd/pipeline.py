@@ -22,8 +22,9 @@ from .types import Buffers
 
 
 def _arr(x):
-    """Device tensors pass through; everything else becomes a numpy array."""
-    if isinstance(x, torch.Tensor):
+    """Device tensors and None (which the library refuses where a shader reads the array)
+    pass through; everything else becomes a numpy array."""
+    if x is None or isinstance(x, torch.Tensor):
         return x
     return np.asarray(x)
 
